@@ -13,7 +13,7 @@ import torch  # noqa: F401  (load order: see module docstring)
 
 LIB_NAME = "libdryft_decode.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -32,6 +32,12 @@ _SIGS = {
     "dd_gemv_add_rmsnorm": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _F, _I, _P, _P, _P]),
     "dd_gemv_add_rmsnorm_ws_bytes": (_Z, [_I, _I, _I, _I]),
     "dd_gate_up_silu": (_I, [_P, _P, _P, _I, _I, _I, _P]),
+    "dd_linear_supported": (_I, [_I, _I, _I]),
+    "dd_linear_ws_bytes": (_Z, [_I, _I, _I]),
+    "dd_linear_counters": (_I, [_I, _I, _I]),
+    "dd_linear": (_I, [_P, _P, _P, _I, _I, _I, _P, _P, _P]),
+    "dd_linear_silu": (_I, [_P, _P, _P, _I, _I, _I, _P, _P, _P]),
+    "dd_linear_add_rmsnorm": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _F, _P, _P, _P]),
     "dd_silu_mul": (_I, [_P, _P, _I, _I, _P]),
     "dd_qkv_post_decode": (_I, [_P, _P, _P, _P, _P, _I, _P, _I, _P, _P, _P,
                                 _I, _I, _I, _I, _I, _I, _F, _P, _P]),

@@ -226,6 +226,38 @@ def test_linear_add_norm_real(small, weights, name):
         close(y, ry)
 
 
+# rows at the edges of the 16-row tiles; N and K at a ragged last tile, tiles of 1 / 2 / 4 / 5 / 8 weight
+# tiles, K split over workgroups (few outputs, many rows) and every stage width
+@pytest.mark.parametrize("M", [1, 16, 17, 48, 64])
+@pytest.mark.parametrize("N,K", [(72, 256), (1000, 192), (2560, 1024), (6144, 128), (20002, 64), (40000, 128)])
+def test_streamed_linear_exact(small, M, N, K):
+    """x and W of -1, 0, 1: every product sum is a whole number of at most K <= 1024 with |sum| < 256
+    (a random walk), exact in fp32 in any order and in bf16."""
+    hip = small[1]
+    g = torch.Generator().manual_seed(M * 7 + N)
+    x = torch.randint(-1, 2, (M, K), generator=g).to(torch.bfloat16)
+    w = torch.randint(-1, 2, (N, K), generator=g).to(torch.bfloat16)
+    ref = x.float() @ w.float().t()
+    assert ref.abs().max() < 256
+    assert hip._linear_plan(x.cuda(), w.cuda()) is not None
+    for _ in range(2):                                      # the counters are left zero
+        assert torch.equal(hip.linear(x.cuda(), w.cuda()).float().cpu(), ref)
+    if N % 2 == 0:
+        gu, up = ref.chunk(2, -1)
+        want = (torch.nn.functional.silu(gu).to(torch.bfloat16).float() * up).to(torch.bfloat16)
+        got = hip.gate_up_silu(x.cuda(), w.cuda()).cpu().float()
+        # silu to one bf16 ulp (another expf): 2^-7 at most; one more from the rounding of the product
+        assert ((got - want.float()).abs() <= 2 ** -6 * want.float().abs() + 1e-30).all()
+    if N <= 4096:
+        h = torch.randint(-64, 65, (M, N), generator=g).to(torch.bfloat16)
+        lnw = torch.ones(N, dtype=torch.bfloat16)
+        hn, y = hip.linear_add_norm(x.cuda(), w.cuda(), h.cuda(), lnw.cuda())
+        want = (h.float() + ref).to(torch.bfloat16).float()
+        assert torch.equal(hn.float().cpu(), want)
+        norm = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + hip.e.eps)
+        assert ((y.float().cpu() - norm).abs() <= 2 ** -8 * norm.abs() + 1e-30).all()
+
+
 def test_linear_dtype_and_layout_fallback(small):
     """test_linear_precision.py:16-27: fp32/fp16/non-contiguous inputs route to F.linear."""
     _, hip, _ = small
