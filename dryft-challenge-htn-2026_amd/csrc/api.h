@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
 #include "../../include/dryft_decode.h"
 
 #define DD_API extern "C" __attribute__((visibility("default")))
@@ -14,6 +15,32 @@ inline bool aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
 
 // Launch result: the error of the last launch on this thread (0 when it went through).
 inline int launch_status() { return (int)hipGetLastError(); }
+
+// Compute units of the current device (0 when it cannot be asked), remembered per device.
+inline int cu_count() {
+  static std::atomic<int> known[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int n = known[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    known[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Lets a kernel use `bytes` of dynamic LDS on the current device; `done` (one per kernel) holds the
+// devices where that has been set.
+inline hipError_t allow_lds(const void* kernel, int bytes, std::atomic<unsigned long long>& done) {
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const unsigned long long bit = 1ull << (dev & 63);
+  if (done.load(std::memory_order_relaxed) & bit) return hipSuccess;
+  const hipError_t r = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (r == hipSuccess) done.fetch_or(bit, std::memory_order_relaxed);
+  return r;
+}
 
 // GEMV launch helpers (gemv.hip): split-K choice, k per split, workspace size, and the launch
 // (h != nullptr selects the residual + RMSNorm epilogue; returns the number of splits).

@@ -353,8 +353,6 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
 // C ABI
 #include "api.h"
 
-#include <atomic>
-
 using namespace dd;
 
 namespace {
@@ -363,18 +361,6 @@ struct Plan {
   int bmt, nt, nv, nout, ntiles, KT, S, C, G;
   size_t ws_bytes;
 };
-
-int cu_count() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    cached[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
 
 // The tiling of one product. N: rows of W (mode SILU: 2 I). Returns false for shapes not taken.
 bool plan_for(int mode, int M, int N, int K, Plan& p) {
@@ -415,8 +401,9 @@ template <int BMT, int NT, int MODE>
 int launch1(const lin::Args& a, int G, hipStream_t stream) {
   using Z = lin::Geo<BMT, NT>;
   auto kern = lin::linear_kernel<BMT, NT, MODE>;
-  static const hipError_t attr = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Z::LDS);
-  if (attr != hipSuccess) return (int)attr;
+  static std::atomic<unsigned long long> done;
+  const hipError_t e = allow_lds((const void*)kern, Z::LDS, done);
+  if (e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(kern, dim3(G), dim3(lin::THREADS), Z::LDS, stream, a);
   return launch_status();
 }

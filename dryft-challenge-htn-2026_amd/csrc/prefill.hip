@@ -40,29 +40,6 @@ constexpr int KB = 32;                 // keys per block
 constexpr int MAXG = 8;                // query heads per kv head
 constexpr int KROW = HD + 8;           // LDS K / V row (elements): 272 bytes
 
-// Max and sum over the lane pairs l, l ^ 16 (rows16) and l, l ^ 32 (rows32) through gfx950's
-// v_permlane16_swap / v_permlane32_swap, VALU operations, instead of the LDS round trip
-// (ds_bpermute) __shfl_xor compiles to. Swapping a register with itself leaves the pair (value of
-// the lower row, value of the upper row) in every lane, so the pair's max or sum needs no
-// lane-dependent select; the sum adds the lower row's value first in every lane, the same bits as
-// either order.
-__device__ __forceinline__ float max_rows16(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float max_rows32(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float sum_rows16(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float sum_rows32(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 // prompt and position of packed token t (seq_start: B + 1 ascending offsets)
 __device__ __forceinline__ void locate(const int* __restrict__ seq_start, int B, int t, int& b, int& p) {
   int lo = 0, hi = B - 1;
@@ -173,16 +150,6 @@ struct FlashShared {
   bf16 k[KB][KROW];                    // the block's keys, row-major
   bf16 v[KB][KROW];                    // the block's values, row-major (read transposed)
 };
-
-// ds_read_b64_tr_b16 (gfx950), a transposing LDS read: when lane (l16, g4) of a wave addresses
-// row g4 * 4 + l16 / 4, columns c0 + 4 (l16 % 4) .. + 3 of a row-major bf16 array, it receives
-// column c0 + l16 of rows g4 * 4 .. g4 * 4 + 3 (the MFMA operand of the transposed block).
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 lds_read_tr16(const bf16* p) {
-  const i16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) i16x4*)(const_cast<bf16*>(p)));
-  return __builtin_bit_cast(u32x2, v);
-}
 
 // Tile index -> (prompt, first token position) for tiles of TQ tokens. ntile[b] = ceil(len_b /
 // TQ); tiles are numbered prompt by prompt, and workgroup x takes tile (total - 1 - x), so the

@@ -119,7 +119,8 @@ int dd_qkv_post_decode(const void* qkv, const void* qn, const void* kn, const vo
 /* Split-KV GQA decode attention with log-sum-exp combine.
  * q: [B, NKV, W, G, HD] (dd_qkv_post_decode layout); kc/vc: [B, NKV, cap, HD] (zero-initialised);
  * query row (b, s) sees keys 0 .. pos[b*pos_stride] + s. out: [B*W, NH*HD].
- * chunk: keys per split (multiple of 32; <= 0 picks dd_attn_chunk). ws: dd_attn_ws_bytes bytes;
+ * chunk: keys per split (multiple of 32; <= 0 picks dd_attn_chunk); with dd_attn_chunk's own value
+ * and W*G <= 4, B <= 512 the batch is dealt in equal shares instead. ws: dd_attn_ws_bytes bytes;
  * counters: B*NKV ints, zero before the first call (kernels leave them zero).
  * HD must be 128 and W*G <= 32.
  * Replaces TritonOps.attn_decode (fused.py:961-987; kernels fused.py:478-565), reference

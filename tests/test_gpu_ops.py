@@ -403,6 +403,31 @@ def test_attn_ragged_long_context(cuda):
     assert d < 0.02, d
 
 
+# equal shares of the batch (W * G <= 4): contexts at the edges of the 32-key blocks, empty and full
+# caches, pairs that lie in one wave, in several, in several workgroups, more pairs than workgroups,
+# a capacity that is no multiple of the block, W = 2
+@pytest.mark.parametrize("NH,NKV,W,cap,lens", [
+    (32, 8, 1, 64, [1]), (32, 8, 1, 64, [64, 1, 33]), (32, 8, 1, 8192, [8192]), (32, 8, 1, 640, [577] * 33),
+    (32, 8, 1, 4100, [4100, 1, 31, 32, 33, 4095, 64, 96]), (4, 4, 1, 200, [7 * i % 199 + 1 for i in range(130)]),
+    (32, 8, 1, 330, [11 * i % 331 for i in range(1, 300)]),
+    (8, 4, 2, 328, [2, 33, 328, 100, 257]), (12, 4, 1, 1000, [999, 3])])
+def test_attn_equal_shares(cuda, NH, NKV, W, cap, lens):
+    HD = 128
+    hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
+    B, g = len(lens), torch.Generator().manual_seed(cap + len(lens))
+    kc, vc = (torch.randn(B, NKV, cap, HD, generator=g).to(BF) for _ in range(2))
+    q = torch.randn(B, NKV, W, NH // NKV, HD, generator=g).to(BF)
+    pos = torch.tensor(lens) - W
+    kg, vg = kc.cuda(), vc.cuda()
+    for b, n in enumerate(lens):                            # the cache is zero past the last key
+        kg[b, :, n:] = vg[b, :, n:] = 0
+    args = q.cuda(), kg, vg, pos.cuda(), W
+    out = hip.attn_decode(*args)
+    assert torch.equal(out, hip.attn_decode(*args))         # same bits, counters left zero
+    d = (out.double().cpu() - attn_reference_fp64(q, kc, vc, pos, W, NH, NKV, HD)).abs().max().item()
+    assert d < 0.02, d
+
+
 # ------------------------------------------------------------------------ argmax
 def test_argmax_rules_and_pos(cuda):
     from dryft_amd.hipops import HipOps
