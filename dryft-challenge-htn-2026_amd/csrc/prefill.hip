@@ -55,7 +55,11 @@ __device__ __forceinline__ void locate(const int* __restrict__ seq_start, int B,
 // One workgroup per 16 tokens: each 16-lane group takes one token's heads in turn, QKV_HPB heads'
 // loads in flight together. Lane j of a group holds dims 4j .. 4j + 3 and 64 + 4j .. 64 + 4j + 3
 // (two 8-byte accesses), so both rotate-half partners of every dim are in the lane; the head's
-// sum of squares is the lane's 8 squares added in order, then reduced over the 16 lanes.
+// sum of squares is the lane's 8 squares added in order, then reduced over the 16 lanes. The heads are
+// split over the grid's second dimension, hpw each: a workgroup's batches of heads are a chain of
+// memory round trips, which is all that a short prompt's pass takes (us, graph-timed, 48 heads: 48 /
+// 8 / 4 per workgroup): 131 tokens 29.4 / 7.4 / 5.2, 512 30.1 / 8.6 / 7.2, 2,048 32.5 / 16.1 / 13.8,
+// 8,192 54.9 / 44.2 / 47.1, 16,223 96.4 / 94.1 / 93.5 (4.3 TB/s; a large copy reaches 4.9).
 constexpr int QKV_TPW = 16;            // tokens per workgroup (4 waves x 4 groups)
 #ifndef DD_QKV_HPB
 #define DD_QKV_HPB 8
@@ -74,7 +78,7 @@ qkv_prefill_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ qn,
                    const bf16* __restrict__ sin_t, const int* __restrict__ seq_start, int B, int T,
                    int last_only, bf16* __restrict__ q_out, bf16* __restrict__ kc,
                    bf16* __restrict__ vc, int NH, int NKV, int cap, int rope_rows, float eps,
-                   int* __restrict__ err) {
+                   int* __restrict__ err, int hpw) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int j = lane & 15;
   const int t = blockIdx.x * QKV_TPW + wave * 4 + (lane >> 4);   // this group's token
@@ -83,12 +87,13 @@ qkv_prefill_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ qn,
   locate(seq_start, B, t, b, p);
   const int len = seq_start[b + 1] - seq_start[b];
   if (p < 0 || p >= len || p >= cap || p >= rope_rows) {   // never write outside the cache
-    if (j == 0 && err != nullptr) atomicOr(err, 2);
+    if (j == 0 && blockIdx.y == 0 && err != nullptr) atomicOr(err, 2);
     return;
   }
   // last_only: q of each prompt's last token only, at row b (the last layer's queries)
-  const int h_first = last_only && p != len - 1 ? NH : 0;
   const int nheads = NH + 2 * NKV;
+  const int h_first = max((int)blockIdx.y * hpw, last_only && p != len - 1 ? NH : 0);
+  const int h_end = min(nheads, ((int)blockIdx.y + 1) * hpw);        // this workgroup's heads
   const int d0 = 4 * j, d1 = 64 + 4 * j;
   const size_t cb = (size_t)p * HD;
   const u32x2 c0 = *(const u32x2*)(cos_t + cb + d0), c1 = *(const u32x2*)(cos_t + cb + d1);
@@ -100,18 +105,18 @@ qkv_prefill_kernel(const bf16* __restrict__ qkv, const bf16* __restrict__ qn,
   const float sw[8] = {lo_bf(s0.x), hi_bf(s0.x), lo_bf(s0.y), hi_bf(s0.y),
                        lo_bf(s1.x), hi_bf(s1.x), lo_bf(s1.y), hi_bf(s1.y)};
   const bf16* row = qkv + (size_t)t * nheads * HD;
-  for (int h0 = h_first; h0 < nheads; h0 += QKV_HPB) {
+  for (int h0 = h_first; h0 < h_end; h0 += QKV_HPB) {
     u32x2 xa[QKV_HPB], xb[QKV_HPB];
 #pragma unroll
     for (int i = 0; i < QKV_HPB; ++i) {
       const int h = h0 + i;
-      xa[i] = h < nheads ? *(const u32x2*)(row + (size_t)h * HD + d0) : u32x2{0u, 0u};
-      xb[i] = h < nheads ? *(const u32x2*)(row + (size_t)h * HD + d1) : u32x2{0u, 0u};
+      xa[i] = h < h_end ? *(const u32x2*)(row + (size_t)h * HD + d0) : u32x2{0u, 0u};
+      xb[i] = h < h_end ? *(const u32x2*)(row + (size_t)h * HD + d1) : u32x2{0u, 0u};
     }
 #pragma unroll
     for (int i = 0; i < QKV_HPB; ++i) {
       const int h = h0 + i;
-      if (h >= nheads) break;
+      if (h >= h_end) break;
       if (h >= NH + NKV) {             // v: a straight copy into the cache
         bf16* dst = vc + (((size_t)b * NKV + (h - NH - NKV)) * cap + p) * HD;
         *(u32x2*)(dst + d0) = xa[i];
@@ -516,10 +521,13 @@ DD_API int dd_qkv_post_prefill(const void* qkv, const void* qn, const void* kn, 
   DD_REQUIRE(HD == 128 && B >= 1 && T >= 1 && NKV >= 1 && NH >= NKV && NH % NKV == 0);
   DD_REQUIRE(cap >= 1 && rope_rows >= 1);
   DD_REQUIRE((long long)T * (NH + 2 * NKV) * HD < (1ll << 40));
-  hipLaunchKernelGGL(pf::qkv_prefill_kernel, dim3((T + pf::QKV_TPW - 1) / pf::QKV_TPW), dim3(256), 0,
+  const int nheads = NH + 2 * NKV;
+  const int hpw = T <= 4096 ? 4 : 8;     // heads per workgroup, see qkv_prefill_kernel
+  hipLaunchKernelGGL(pf::qkv_prefill_kernel,
+                     dim3((T + pf::QKV_TPW - 1) / pf::QKV_TPW, (nheads + hpw - 1) / hpw), dim3(256), 0,
                      stream, (const bf16*)qkv, (const bf16*)qn, (const bf16*)kn, (const bf16*)cos_t,
                      (const bf16*)sin_t, seq_start, B, T, last_only, (bf16*)q_out, (bf16*)kc,
-                     (bf16*)vc, NH, NKV, cap, rope_rows, eps, err);
+                     (bf16*)vc, NH, NKV, cap, rope_rows, eps, err, hpw);
   return launch_status();
 }
 
