@@ -25,8 +25,7 @@
 // O^T += V^T.P^T; the key order inside each P.V contraction is the one each lane's S^T
 // accumulators hold, so P never leaves the lane. A wave skips the blocks past its last token.
 // Tiles holding a prompt's last tokens (the longest causal prefixes) are scheduled first.
-// flash_prefill_dma_kernel: the same arithmetic for G = 4 with one query head per wave, its
-// 32-key blocks staged by LDS-DMA loads into two swizzled LDS buffers (the G = 4 default).
+// flash_prefill_pp_kernel: G = 4 with 32 queries per wave and 64-key blocks staged by LDS-DMA loads.
 #include <type_traits>
 
 #include "common.h"
@@ -190,9 +189,6 @@ __device__ __forceinline__ bool tile_of(const int* __restrict__ seq_start, int B
 // q [T, NH, HD] token-major; out [T, NH * HD] (last_only: [B, NH, HD] / [B, NH * HD], row b =
 // prompt b's last token). HPW query heads per wave, NTT 16-token tiles per workgroup, with
 // NTT * (NH / NKV) / HPW = NWAVE_F waves; MINB workgroups per CU (the register budget).
-#ifndef DD_PF_MINB1
-#define DD_PF_MINB1 4
-#endif
 #ifndef DD_PF_MINB
 #define DD_PF_MINB 2
 #endif
@@ -354,154 +350,290 @@ flash_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc, co
   }
 }
 
-// The same attention (one query head per wave, 16 tokens, G = 4 waves per workgroup) with the
-// 32-key blocks staged by LDS-DMA loads (buffer_load_dwordx4 ... lds: lane i's 16 bytes land at
-// the wave's LDS base + 16 i) into two buffers: block j + 1 streams into one while block j is
-// read from the other, with one barrier per block and no staging registers. Rows are 256 bytes,
-// unpadded; 16-byte chunks are XOR-swizzled so that the MFMA operand reads meet distinct banks:
-// K chunk c of key r at position c ^ (r % 16) (a K read: 16 consecutive keys, one chunk), V chunk
-// c of key r at c ^ 2 (r % 8) (a transposing V read: 4 consecutive keys, a pair of chunks).
-// The DMA writer picks, per lane, the source chunk whose swizzled position is its own. The loop is
-// unrolled by two so each buffer is a separate LDS object at every access.
-struct FlashDmaBuf {
-  bf16 k[KB * HD];
-  bf16 v[KB * HD];
-};
+// ---------------------------------------------------------------------------------------------
+// The same attention for G = 4 with 32 queries per wave and 64-key blocks: wave w takes query head w % 4 of
+// tokens 32 (w / 4) .. + 31 of its workgroup's tile, 8 waves (64 tokens, one workgroup per CU) or 4 (32
+// tokens, two per CU).
+//
+// What bounds it: MFMA and the softmax's VALU work are about equal (per wave and block 32 MFMAs of
+// 32x32x16, 1,024 cycles, against ~220 VALU instructions), and every K / V operand byte read from LDS
+// feeds 32 queries (16 in the kernel above). So the two waves of a SIMD should be in different parts of
+// a block: two workgroups of 4 waves are by themselves; the halves of an 8-wave workgroup (waves w and
+// w + 4 share a SIMD) run one phase apart: while waves 0 - 3 multiply (P.V of block j and K.Q of block
+// j + 1), waves 4 - 7 do the softmax of block j, then the other way round, one barrier a phase. S and P
+// of one block are all that a wave holds. K and V have 3 LDS buffers each (2 for 4 waves), filled by
+// LDS-DMA four phases (a block) ahead; asm, so that the compiler ties no LDS read to the loads in
+// flight; the waits are made by hand. The operand reads of a phase run ahead of its MFMAs (left in the
+// compiler's order 671 against 617 us at 8,192 tokens). The kv head is the grid's fast dimension: the
+// heaviest tiles of every head go first (with the tiles fast, the last head's heavy tiles started last:
+// 617 against 527 us), and each XCD's L2 sees the keys of NKV / 8 heads.
+// A query's bits do not depend on the tile or the number of waves.
+//
+// Graph-timed on MI355X, us, with 16 queries per wave and 32-key blocks (the kernel that this one
+// replaced) / 4 waves / 8 waves: 131 tokens 8.2 / 9.3 / 12.2, 512 17.0 / 16.7 / 21.9, 1,000 33.4 / 27.7 /
+// 32.6, 2,048 91.6 / 57.6 / 63.5, 16 prompts of 64 - 2,048 346 / 292 / 302, 4,096 - / 174 / 157, 8,192 770 /
+// 549 / 525 (1.05 PFLOP/s of causal attention; MFMA 52% busy at the 1.9 GHz that the card holds): 8
+// waves from 4,096 tokens per prompt on.
+//
+// 32x32x16 layouts: S^T lane l holds query l % 32, keys 8 (i / 4) + 4 (l / 32) + i % 4 of 32; those are
+// the keys its P values keep in the P.V contraction, so P never leaves the lane and the V^T operand
+// reads (transposing) fetch those keys. LDS rows are 256 bytes, 16-byte chunk c of row r at c ^ (r % 16)
+// for K (an operand read: one chunk of 32 rows), c ^ 4 (r % 4) for V (4 rows, 4 chunks a half wave):
+// no bank conflicts counted.
+constexpr int PP_KB = 64;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-template <int MINB>
-__global__ void __launch_bounds__(256, MINB)
-flash_prefill_dma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
-                         const int* __restrict__ seq_start, int B, int T, bf16* __restrict__ out,
-                         int NH, int NKV, int cap, int last_only, float scale_log2) {
-  __shared__ __attribute__((aligned(16))) FlashDmaBuf sb0;
-  __shared__ __attribute__((aligned(16))) FlashDmaBuf sb1;
-  constexpr int TQ = 16;
+// LDS bytes: 3 buffers of K and of V for 8 waves, 2 for 4
+constexpr int pp_lds(int nw) { return (nw == 8 ? 3 : 2) * 2 * PP_KB * HD * 2; }
+
+__device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
+}
+
+template <int NW>
+__global__ void __launch_bounds__(64 * NW, 2)
+flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
+                        const int* __restrict__ seq_start, int B, int T, bf16* __restrict__ out, int NH, int NKV,
+                        int cap, int last_only, float scale_log2) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char pp_smem[];
+  constexpr int TQ = 8 * NW, G = 4, NB = NW == 8 ? 3 : 2, BUF = PP_KB * HD, IPW = 16 / NW;
+  bf16* const shk = (bf16*)pp_smem;
+  bf16* const shv = shk + NB * BUF;
   int b = 0, p0 = 0;
-  if (!tile_of(seq_start, B, blockIdx.x, last_only != 0, TQ, b, p0)) return;
-  const int G = NH / NKV, kvh = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int l16 = lane & 15, g4 = lane >> 4;
-  const int head = kvh * G + wave;                              // this wave's query head
+  if (!tile_of(seq_start, B, blockIdx.y, last_only != 0, TQ, b, p0)) return;
+  const int kvh = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31, h = lane >> 5;
+  const bool late = wave >= 4;                                  // one phase behind (waves w, w + 4 share a SIMD)
+  const int head = kvh * G + (wave & 3);
   const int s0 = seq_start[b], len = seq_start[b + 1] - s0;
   if (s0 < 0 || len <= 0 || s0 + len > T || len > cap) return;   // inconsistent offsets: no access
-  const int pq = p0 + l16;                                      // this lane's query token position
+  const int pq = p0 + (late ? 32 : 0) + l32;                    // this lane's query position
   const bool qok = last_only ? pq == len - 1 : pq < len;
-  const bool wact = last_only ? (len - 1 >= p0 && len - 1 < p0 + 16) : p0 < len;
-  const int wlast = min(p0 + 15, len - 1);
-  const int nblk = wlast / KB + 1;
-  u32x4 qreg[4];
+  const size_t qrow = last_only ? b : s0 + pq;
+  const int nblk = (min(p0 + TQ, len) - 1) / PP_KB + 1;
+  u32x4 qreg[8];
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb)
-    qreg[kb] = qok ? *(const u32x4*)(q + ((size_t)(last_only ? b : s0 + pq) * NH + head) * HD + kb * 32 + g4 * 8)
-                   : u32x4{0u, 0u, 0u, 0u};
-  f32x4 acc[8];
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  for (int ks = 0; ks < 8; ++ks)
+    qreg[ks] = qok ? *(const u32x4*)(q + (qrow * NH + head) * HD + ks * 16 + h * 8) : u32x4{0u, 0u, 0u, 0u};
   const size_t kvbase = ((size_t)b * NKV + kvh) * cap * HD;
-  const rsrc_t kr = make_rsrc(kc + kvbase, (unsigned)((size_t)cap * HD * 2));
-  const rsrc_t vr = make_rsrc(vc + kvbase, (unsigned)((size_t)cap * HD * 2));
-  // DMA: wave w writes LDS positions (2 w + j) 64 + lane (16-byte chunks) of each matrix
-  unsigned koff[2], voff[2];
+  const rsrc_t kr = make_rsrc(kc + kvbase, (unsigned)len * HD * 2), vr = make_rsrc(vc + kvbase, (unsigned)len * HD * 2);
+  const unsigned lds_k = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) bf16*)shk);
+  const unsigned lds_v = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) bf16*)shv);
+  // DMA: instruction i fills rows 4 i .. 4 i + 3 of a buffer; wave w issues IPW of them. Rows past the
+  // prompt repeat its last key (masked); blocks past the last repeat it (not used).
+  auto dma = [&](rsrc_t r, unsigned voff, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds) : "memory");
+  };
+  const int drow = 4 * IPW * wave + (lane >> 4), dc = lane & 15;
+  auto issue_k = [&](int j, int buf) {
+    const int key0 = min(j, nblk - 1) * PP_KB;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int p = (2 * wave + j) * 64 + lane, r = p >> 4, c = p & 15;
-    koff[j] = (unsigned)(r * HD * 2 + ((c ^ (r & 15)) * 16));
-    voff[j] = (unsigned)(r * HD * 2 + ((c ^ (2 * (r & 7))) * 16));
-  }
-  typedef __attribute__((address_space(3))) void* lds_t;
-  auto issue = [&](FlashDmaBuf& s, int key0) {
-    const unsigned so = (unsigned)key0 * HD * 2;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (lds_t)&s.k[(2 * wave + j) * 512], 16, koff[j], so, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (lds_t)&s.v[(2 * wave + j) * 512], 16, voff[j], so, 0, 0);
+    for (int i = 0; i < IPW; ++i) {
+      const int r = drow + 4 * i;
+      dma(kr, (unsigned)min(key0 + r, len - 1) * HD * 2 + (dc ^ (r & 15)) * 16, lds_k + buf * (BUF * 2) + (IPW * wave + i) * 1024);
     }
   };
-  // MFMA operand addresses (elements) inside a buffer
-  int ka_off[2][4];
+  auto issue_v = [&](int j, int buf) {
+    const int key0 = min(j, nblk - 1) * PP_KB;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const int r = t * 16 + l16, c = kb * 4 + g4;
-      ka_off[t][kb] = r * HD + ((c ^ (r & 15)) << 3);
+    for (int i = 0; i < IPW; ++i) {
+      const int r = drow + 4 * i;
+      dma(vr, (unsigned)min(key0 + r, len - 1) * HD * 2 + (dc ^ (4 * (r & 3))) * 16, lds_v + buf * (BUF * 2) + (IPW * wave + i) * 1024);
     }
-  const int trow = g4 * 4 + (l16 >> 2), tcol = 4 * (l16 & 3);
-  int vt_off[2][8];
+  };
+  auto phase_end = [&] {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto landed = [&] {                                           // all but this wave's latest 4 loads
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  };
+  // operand addresses (elements) inside a buffer
+  int ka[8], va[4];
 #pragma unroll
-  for (int hh = 0; hh < 2; ++hh)
+  for (int ks = 0; ks < 8; ++ks) ka[ks] = l32 * HD + (((ks * 2 + h) ^ (l32 & 15)) << 3);
+  {
+    const int l16 = lane & 15, g = (lane >> 4) & 1, r = 4 * h + (l16 >> 2);
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const int r = hh * 16 + trow, col = dt * 16 + tcol;
-      vt_off[hh][dt] = r * HD + ((((col >> 3) ^ (2 * (r & 7)))) << 3) + (col & 7);
+    for (int d = 0; d < 4; ++d) {
+      const int col = d * 32 + g * 16 + 4 * (l16 & 3);
+      va[d] = r * HD + (((col >> 3) ^ (4 * (r & 3))) << 3) + (col & 7);
     }
-  const int nfull = min(nblk, (p0 + 1) / KB);                  // blocks that need no causal mask
-  // one block: wait for its DMA (this wave's, then every wave's through the barrier), start the
-  // next block's DMA into the other buffer (free: every wave is past its previous block), then
-  // (the wave's keys permitting) add it
-  auto block = [&](const FlashDmaBuf& cur, FlashDmaBuf& nxt, int blk) {
-    const int key0 = blk * KB;
-    __builtin_amdgcn_s_waitcnt(0x0f70);                        // vmcnt(0)
-    __syncthreads();
-    if (blk + 1 < nblk) issue(nxt, key0 + KB);
-    if (!wact || key0 > wlast) return;                          // wave-uniform: nothing to add
-    const bool masked = blk >= nfull;
-    f32x4 sc[2];
+  }
+  f32x16 acc[4], sc[2];
+  u32x4 pk[4];
+  float m_run = -INFINITY, l_run = 0.f;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[d][i] = 0.f;
+  auto qk = [&](int buf) {                                      // S^T of a block
+    const bf16* kb = shk + buf * BUF;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      f32x4 d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) d = mfma16x16x32(*(const u32x4*)&cur.k[ka_off[t][kb]], qreg[kb], d);
-      sc[t] = d;
+      for (int i = 0; i < 16; ++i) sc[t][i] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) sc[t] = mfma32(*(const u32x4*)&kb[t * 32 * HD + ka[ks]], qreg[ks], sc[t]);
     }
-    float sv[8];
-    float mloc = -INFINITY;
+  };
+  // O^T += V^T.P^T of a block, and (QK) S^T of the next one. The operand reads run two key steps ahead of
+  // their MFMAs: left alone, the compiler reads each operand right before its MFMA and waits for it.
+  auto pv = [&](int bv, int bk, auto with_qk) {
+    constexpr bool QK = decltype(with_qk)::value;
+    const bf16* vb = shv + bv * BUF;
+    u32x4 vf[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const u32x2 lo = lds_read_tr16(&vb[t * 16 * HD + va[d]]);
+        const u32x2 hi = lds_read_tr16(&vb[(t * 16 + 8) * HD + va[d]]);
+        vf[t][d] = u32x4{lo.x, lo.y, hi.x, hi.y};
+      }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) acc[d] = mfma32(vf[t][d], pk[t], acc[d]);
+    if constexpr (QK) qk(bk);
+    __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);         // V of steps 0 and 1
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);        // V of steps 2 and 3
+    }
+    if constexpr (QK) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);      // K
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+    } else {
+      __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    }
+  };
+  auto softmax = [&](int j) {
+    if (j * PP_KB + PP_KB - 1 > p0 + (late ? 32 : 0)) {         // the block reaches past the wave's first query
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (j * PP_KB + t * 32 + 8 * (i / 4) + 4 * h + i % 4 > pq) sc[t][i] = -INFINITY;
+    }
+    float mx = -INFINITY;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = key0 + t * 16 + g4 * 4 + i;
-        const float v = !masked || (qok && key <= pq) ? sc[t][i] * scale_log2 : -INFINITY;
-        sv[t * 4 + i] = v;
-        mloc = fmaxf(mloc, v);
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[t][i]);
+    mx = max_rows32(mx);                                        // raw scores
+    const bool up = mx > m_run;                                 // the first block: key 0 is always seen
+    if (__any(up)) {
+      const float m_new = up ? mx : m_run;
+      const float alpha = exp2_hw((m_run - m_new) * scale_log2);   // 1 in rows that keep theirs
+      l_run *= alpha;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] *= alpha;
+      m_run = m_new;
+    }
+    const float mscl = m_run * scale_log2;
+    float ps[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        const float pa = exp2_hw(__builtin_fmaf(sc[t][i], scale_log2, -mscl));
+        const float pb = exp2_hw(__builtin_fmaf(sc[t][i + 1], scale_log2, -mscl));
+        ps[(i / 2) & 3] += pa + pb;
+        pk[t * 2 + i / 8][(i & 7) / 2] = pk_bf16(pa, pb);
       }
-    mloc = max_rows32(max_rows16(mloc));
-    const float m_new = fmaxf(m_run, mloc);
-    const float msafe = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = exp2_hw(m_run - msafe);
-    float psum = 0.f;
-    unsigned pk[4];
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const float pa = exp2_hw(sv[2 * jj] - msafe);
-      const float pb = exp2_hw(sv[2 * jj + 1] - msafe);
-      psum += pa + pb;
-      pk[jj] = pk_bf16(pa, pb);
-    }
-    psum = sum_rows32(sum_rows16(psum));
-    l_run = l_run * alpha + psum;
-    m_run = m_new;
-    const u32x4 pB = {pk[0], pk[1], pk[2], pk[3]};
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const u32x2 lo = lds_read_tr16(&cur.v[vt_off[0][dt]]);
-      const u32x2 hi = lds_read_tr16(&cur.v[vt_off[1][dt]]);
-      acc[dt] *= alpha;
-      acc[dt] = mfma16x16x32(u32x4{lo.x, lo.y, hi.x, hi.y}, pB, acc[dt]);
-    }
+    l_run += sum_rows32((ps[0] + ps[1]) + (ps[2] + ps[3]));
   };
-  issue(sb0, 0);
-  for (int blk = 0; blk < nblk; blk += 2) {
-    block(sb0, sb1, blk);
-    if (blk + 1 < nblk) block(sb1, sb0, blk + 1);
+
+  const std::integral_constant<bool, true> next{};
+  const std::integral_constant<bool, false> final{};
+  issue_k(0, 0);
+  issue_k(1, 1);
+  issue_v(0, 0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  phase_end();
+  if constexpr (NW == 4) {                                      // two workgroups per CU overlap by themselves
+    qk(0);
+    for (int j = 0; j + 1 < nblk; ++j) {
+      softmax(j);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      phase_end();                                              // block j - 1 is read, V(j) and K(j + 1) landed
+      issue_k(j + 2, j & 1);
+      issue_v(j + 1, (j + 1) & 1);
+      pv(j & 1, (j + 1) & 1, next);
+    }
+    softmax(nblk - 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    phase_end();
+    pv((nblk - 1) & 1, 0, final);
+  } else {
+    issue_k(2, 2);
+    issue_v(1, 1);
+    int b0 = 0, b1 = 1, b2 = 2;                                   // buffers of blocks j, j + 1, j + 2 (K and V)
+    auto turn = [&] {
+      const int t = b0;
+      b0 = b1;
+      b1 = b2;
+      b2 = t;
+    };
+    if (!late) {
+      qk(0);
+      phase_end();
+      for (int j = 0; j + 1 < nblk; ++j) {
+        softmax(j);
+        landed();
+        phase_end();
+        issue_k(j + 3, b0);
+        issue_v(j + 2, b2);
+        pv(b0, b1, next);
+        phase_end();
+        turn();
+      }
+      softmax(nblk - 1);
+      landed();
+      phase_end();
+      pv(b0, b1, final);
+      phase_end();
+    } else {
+      phase_end();
+      qk(0);
+      landed();
+      phase_end();
+      for (int j = 0; j + 1 < nblk; ++j) {
+        issue_k(j + 3, b0);
+        issue_v(j + 2, b2);
+        softmax(j);
+        phase_end();
+        pv(b0, b1, next);
+        landed();
+        phase_end();
+        turn();
+      }
+      softmax(nblk - 1);
+      phase_end();
+      pv(b0, b1, final);
+    }
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // no load into LDS outlives the wave
   if (!qok) return;
-  bf16* orow = last_only ? out + ((size_t)b * NH + head) * HD : out + ((size_t)(s0 + pq) * NH + head) * HD;
+  const float inv = 1.0f / l_run;
+  bf16* orow = out + (qrow * NH + head) * HD;
 #pragma unroll
-  for (int dt = 0; dt < 8; ++dt)
+  for (int d = 0; d < 4; ++d)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) orow[dt * 16 + g4 * 4 + i] = f2bf(acc[dt][i] / l_run);
+    for (int i = 0; i < 16; i += 4)
+      *(u32x2*)(orow + d * 32 + 2 * i + 4 * h) = u32x2{pk_bf16(acc[d][i] * inv, acc[d][i + 1] * inv),
+                                                      pk_bf16(acc[d][i + 2] * inv, acc[d][i + 3] * inv)};
 }
 
 }  // namespace pf
@@ -549,27 +681,23 @@ DD_API int dd_attn_prefill(const void* q, const void* kc, const void* vc, const 
                        (const bf16*)kc, (const bf16*)vc, seq_start, B, T, (bf16*)out, NH, NKV, cap,
                        last_only, scale_log2);
   };
+  hipError_t attr = hipSuccess;
+  auto launch_pp = [&](int nw) {
+    static std::atomic<unsigned long long> done4, done8;
+    auto kern = nw == 8 ? pf::flash_prefill_pp_kernel<8> : pf::flash_prefill_pp_kernel<4>;
+    attr = allow_lds((const void*)kern, pf::pp_lds(nw), nw == 8 ? done8 : done4);
+    if (attr != hipSuccess) return;
+    const int ntiles = last_only ? B : T / (8 * nw) + B;
+    hipLaunchKernelGGL(kern, dim3(NKV, ntiles), dim3(64 * nw), pf::pp_lds(nw), stream, (const bf16*)q, (const bf16*)kc,
+                       (const bf16*)vc, seq_start, B, T, (bf16*)out, NH, NKV, cap, last_only, scale_log2);
+  };
   switch (G) {
     case 1: launch(pf::flash_prefill_kernel<1, 4, 4, DD_PF_MINB>, 64, 4); break;
     case 2: launch(pf::flash_prefill_kernel<2, 4, 4, DD_PF_MINB>, 64, 4); break;
-// G = 4 (Qwen3): one query head per wave, 16 tokens per workgroup, four workgroups per CU (four
-// waves per SIMD). configs[4]'s packed prompts, one process alternating builds, us per layer, the
-// same bits throughout: two heads per wave (211 VGPRs, two workgroups per CU) 368; one head per
-// wave with register staging (108 VGPRs) 338; with the LDS-DMA double buffer (116 VGPRs, 32 KB
-// of LDS) 314-322 against 347-354 on the same boxes. Eight waves per workgroup (32 tokens, half
-// the barriers and DMA issues per token) 370, with the DMA double buffer 353 against 320; five or
-// six workgroups per CU spill (349 with DMA; 676 / 805 without). The DMA kernel's last
-// block may reach past a prompt's keys but not past the cache: it needs cap % 32 == 0 (the
-// engine's capacities are multiples of 128), else the register-staged kernel runs.
-#ifndef DD_PF_G4
-#define DD_PF_G4 5
-#endif
     case 4:
-      if (DD_PF_G4 == 5 && cap % pf::KB == 0) launch(pf::flash_prefill_dma_kernel<DD_PF_MINB1>, 16, 4);
-      else if (DD_PF_G4 == 2) launch(pf::flash_prefill_kernel<2, 2, 4, DD_PF_MINB>, 32, 4);
-      else launch(pf::flash_prefill_kernel<1, 1, 4, DD_PF_MINB1>, 16, 4);
+      launch_pp(!last_only && T / B >= 4096 ? 8 : 4);
       break;
     default: launch(pf::flash_prefill_kernel<2, 1, 4, DD_PF_MINB>, 16, 4); break;   // G = 8
   }
-  return launch_status();
+  return attr != hipSuccess ? (int)attr : launch_status();
 }
