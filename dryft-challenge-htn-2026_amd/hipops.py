@@ -14,8 +14,8 @@ Every decode-step method calls the C ABI on torch's current stream; outputs and 
 allocated with ``torch.empty`` (so they come from the graph pool under capture). A nonzero
 status raises ``RuntimeError``.
 """
+import bisect
 import json
-import math
 import os
 
 import torch
@@ -26,7 +26,9 @@ from ._lib import check, lib
 BM_MAX = 16  # largest activation-row count the skinny GEMV takes (fused.py:838 BM_MAX role)
 LIN_MAX = 64  # largest activation-row count of the weight-streaming linear kernels
 NORM_MAX = 4096  # longest row the row-norm kernels take
-GEMM_MIN_M = 256  # smallest row count sent to the tuned hipBLASLt GEMM (prefill-sized products)
+# Smallest row count sent to the library's own hipBLASLt call: everything past the skinny kernels.
+# (F.linear asks hipBLASLt's heuristic again on every call, 21 us of host time against 6.)
+GEMM_MIN_M = LIN_MAX + 1
 
 
 def _ptr(t):
@@ -53,18 +55,20 @@ def load_gemm_table(path=GEMM_TABLE):
 
 
 def gemm_solution(table, N, K, M):
-    """The table's solution for an (N, K) product of M rows: the entry whose row count is
-    nearest to M on a log scale (the smaller on a tie), or -1 (heuristic first) for shapes the
-    table lacks."""
+    """The table's solution for an (N, K) product of M rows: the entry of the smallest row count
+    that is not below M (a product's time is a staircase in M, its steps the tile heights; the
+    largest entry above the table), or -1 (heuristic first) for shapes the table lacks."""
     rows = table.get((N, K))
     if not rows:
         return -1
-    lm = math.log(M)
-    return min(rows, key=lambda r: abs(math.log(r[0]) - lm))[1]
+    return rows[min(bisect.bisect_left(rows, (M,)), len(rows) - 1)][1]
 
 
 def _stream(dev):
-    return torch.cuda.current_stream(dev).cuda_stream
+    """torch's current stream on dev, as the raw pointer (torch.cuda.current_stream builds a Stream
+    object around it: 4.5 us a launch, a third of a small launch's host time)."""
+    i = dev.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
 
 
 def _bf16_ok(*ts):

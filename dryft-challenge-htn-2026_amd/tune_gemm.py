@@ -4,20 +4,17 @@ The prefill's projections run on hipBLASLt (dd_gemm_bf16), whose first heuristic
 up to 40% slower than its best candidate at some Qwen3-4B shapes and row counts. The table fixes
 one hipBLASLt solution per (N, K) and row count, chosen here by timing, so that the engine never
 times at run time and every process computes the same bits for the same prompts. At run time a
-product of M rows takes the entry whose row count is nearest to M on a log scale.
+product of M rows takes the entry of the smallest row count that is not below M.
 
-The grid has four row counts per octave from 256 to 32768. For grid point i the candidates are
-the heuristic's lists (dd_gemm_bf16_solutions) at points i-1, i and i+1, those that support all
-three (dd_gemm_bf16_supported), and the heuristic's own first candidate at each point (entry
--1); each is timed at the three points and the entry is the one whose worst ratio to the best
-time at each point is least, so a row count between grid points is served well too. A timing: one warm-up run, then the least of three runs each after a 512 MB fill
-(twice the last-level cache: every run starts with cold caches, as a prefill GEMM does between
-the pass's other kernels).
-
-The timings are jagged in M (a candidate best at one row count can be 30% off the best a
-fifth of an octave away), so row counts a workload is known to run are added as exact entries
-(--exact, by default the prefills of BASELINE.json's configs[4]: its 16 prompts, 16,223 tokens,
-and its first 8, 8,115 tokens): there the entry is the fastest candidate at exactly that M.
+The grid has the multiples of 64 rows up to 2,048, of 128 up to 20,480 and of 256 up to 32,768: a
+product's time is a staircase in the row count whose steps are the candidates' tile heights (64 to
+256 rows), so the next grid point above M has M's own tile counts. The candidates at a grid point
+are the heuristic's lists (dd_gemm_bf16_solutions) at it and its neighbours, those that support it
+(dd_gemm_bf16_supported), and the heuristic's own first candidate (entry -1); the entry is the
+fastest. A timing: one warm-up run, then the least of three runs each after a 512 MB fill (twice
+the last-level cache: every run starts with cold caches, as a prefill GEMM does between the pass's
+other kernels). Row counts a workload is known to run are added as exact entries (--exact, by
+default the prefills of 16 prompts of 64 - 2,048 tokens, 16,223 tokens, and of the first 8, 8,115).
 
   python3 dryft-challenge-htn-2026_amd/tune_gemm.py [--out PATH] [--exact M ...] [--check M ...]
 
@@ -34,8 +31,19 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HERE = os.path.dirname(os.path.abspath(__file__))
 # Qwen3-4B prefill GEMMs (N, K): fused QKV, O, fused gate/up, down
 SHAPES = {"qkv": (6144, 2560), "o": (2560, 4096), "gate_up": (19456, 2560), "down": (2560, 9728)}
-GRID = sorted({int(round(256 * 2 ** (j / 4) / 16)) * 16 for j in range(29)})
+GRID = sorted({*range(64, 2049, 64), *range(2048, 20481, 128), *range(20480, 32769, 256)})
 FLUSH = 512 << 20
+
+
+def dumps(table):
+    """The table as JSON, one shape's rows or timings to a line."""
+    head = {k: v for k, v in table.items() if k not in ("shapes", "timing_ms", "check")}
+    out = json.dumps(head)[:-1]
+    for part in ("shapes", "timing_ms", "check"):
+        rows = ",\n".join(f"  {json.dumps(k)}: {json.dumps(v, separators=(',', ':'))}"
+                          for k, v in table[part].items())
+        out += f",\n {json.dumps(part)}: {{\n{rows}\n }}"
+    return out + "\n}\n"
 
 
 def main():
@@ -105,28 +113,22 @@ def main():
         lists = {M: listed(N, K, M) for M in GRID}
         rows, tms = [], {}
         for i, M in enumerate(GRID):
-            pts = GRID[max(0, i - 1):i + 2]
-            cands = sorted({s for p in pts for s in lists[p]})
-            cands = [s for s in cands
-                     if all(L.dd_gemm_bf16_supported(p, N, K, ws.numel(), s) for p in pts)]
-            cands.append(-1)             # the heuristic's first candidate at each row count
-            best_at = {p: min(timed(N, K, p, s) for s in lists[p]) for p in pts}
-            score = {s: max(timed(N, K, p, s) / best_at[p] for p in pts) for s in cands}
-            sol = min(score, key=lambda s: (score[s], s != -1, s))
+            near = GRID[max(0, i - 1):i + 2]
+            cands = sorted({s for p in near for s in lists[p]})
+            cands = [s for s in cands if L.dd_gemm_bf16_supported(M, N, K, ws.numel(), s)]
+            cands.append(-1)             # the heuristic's first candidate
+            sol = min(cands, key=lambda s: (timed(N, K, M, s), s != -1, s))
             rows.append([M, sol])
             t, first = timed(N, K, M, sol), timed(N, K, M, -1)
-            tms[str(M)] = {"table": round(t, 4), "best": round(best_at[M], 4),
-                           "heuristic_first": round(first, 4), "worst_ratio": round(score[sol], 3)}
-            print(f"[tune] {name} {N}x{K} M={M}: solution {sol} {t:.3f} ms (best {best_at[M]:.3f}, "
-                  f"heuristic first {first:.3f}; worst ratio over neighbours {score[sol]:.3f})",
-                  flush=True)
+            tms[str(M)] = {"table": round(t, 4), "heuristic_first": round(first, 4)}
+            print(f"[tune] {name} {N}x{K} M={M}: solution {sol} {t:.3f} ms (heuristic first "
+                  f"{first:.3f})", flush=True)
         for M in args.exact:
             cands = listed(N, K, M)
             sol = min(cands, key=lambda s: (timed(N, K, M, s), s))
             rows.append([M, sol])
             t, first = timed(N, K, M, sol), timed(N, K, M, -1)
-            tms[str(M)] = {"table": round(t, 4), "best": round(t, 4), "heuristic_first": round(first, 4),
-                           "exact": True}
+            tms[str(M)] = {"table": round(t, 4), "heuristic_first": round(first, 4), "exact": True}
             print(f"[tune] {name} {N}x{K} M={M} (exact): solution {sol} {t:.3f} ms (heuristic "
                   f"first {first:.3f})", flush=True)
         rows.sort()
@@ -147,7 +149,7 @@ def main():
                   f"ms, heuristic first {first:.3f} ms", flush=True)
     table["check"] = checks
     with open(args.out, "w") as f:
-        json.dump(table, f, indent=1)
+        f.write(dumps(table))
     print(f"[tune] wrote {args.out}", flush=True)
 
 
