@@ -41,6 +41,15 @@ __device__ __forceinline__ unsigned e4m3(float x) {
   return sign | (unsigned)((e + 7) << 3) | ((r >> 20) & 7u);
 }
 
+// The same bits from the hardware's conversion (v_cvt_pk_fp8_f32, two values an instruction, round to
+// nearest even, OCP e4m3 on gfx950) for magnitudes up to 448: the integer form above costs ~12 VALU
+// instructions a value, which bounded the pass (10.5 M values: quantisation 19.4 us in all, with the
+// hardware's conversion 14.3; 41.9 M 50.9, 41.4).
+__device__ __forceinline__ unsigned e4m3x4(float a, float b, float c, float d) {
+  const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+  return (unsigned)__builtin_amdgcn_cvt_pk_fp8_f32(c, d, lo, true);
+}
+
 __global__ void __launch_bounds__(THREADS)
 amax_kernel(const u32x4* __restrict__ x, size_t n8, float* __restrict__ partials) {
   __shared__ float red[THREADS / 64];
@@ -75,14 +84,21 @@ quant_kernel(const u32x4* __restrict__ x, size_t n8, const float* __restrict__ p
   amax = nanmax(amax, 1e-6f);
   const float inv = 448.0f / amax;
   if (blockIdx.x == 0 && threadIdx.x == 0) scale[0] = amax / 448.0f;
+  const bool finite = amax < INFINITY;                      // then |x * inv| <= 448 (1 + 2^-23) for every x
   for (size_t i = blockIdx.x * (size_t)THREADS + threadIdx.x; i < n8; i += (size_t)gridDim.x * THREADS) {
     const u32x4 v = x[i];
     const unsigned w[4] = {v.x, v.y, v.z, v.w};
-    unsigned q[4];
+    unsigned q[2];
+    if (finite) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      q[j] = e4m3(lo_bf(w[j]) * inv) | (e4m3(hi_bf(w[j]) * inv) << 8);
-    out[i] = make_uint2(q[0] | (q[1] << 16), q[2] | (q[3] << 16));
+      for (int j = 0; j < 2; ++j) q[j] = e4m3x4(lo_bf(w[2 * j]) * inv, hi_bf(w[2 * j]) * inv, lo_bf(w[2 * j + 1]) * inv, hi_bf(w[2 * j + 1]) * inv);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        q[j] = e4m3(lo_bf(w[2 * j]) * inv) | (e4m3(hi_bf(w[2 * j]) * inv) << 8) | (e4m3(lo_bf(w[2 * j + 1]) * inv) << 16) |
+               (e4m3(hi_bf(w[2 * j + 1]) * inv) << 24);
+    }
+    out[i] = make_uint2(q[0], q[1]);
   }
 }
 

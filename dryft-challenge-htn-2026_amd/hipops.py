@@ -15,6 +15,7 @@ allocated with ``torch.empty`` (so they come from the graph pool under capture).
 status raises ``RuntimeError``.
 """
 import bisect
+import functools
 import json
 import os
 
@@ -39,9 +40,10 @@ def _ptr(t):
 GEMM_TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gemm_solutions.json")
 
 
+@functools.lru_cache(maxsize=4)
 def load_gemm_table(path=GEMM_TABLE):
     """{(N, K): [(M, solution), ...] sorted by M} from the committed table, or {} when it is
-    absent (every shape then runs hipBLASLt's first heuristic candidate)."""
+    absent (every shape then runs hipBLASLt's first heuristic candidate). Read once per process."""
     try:
         with open(path) as f:
             doc = json.load(f)
