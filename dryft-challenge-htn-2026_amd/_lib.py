@@ -33,11 +33,10 @@ _SIGS = {
     "dd_gemv_add_rmsnorm_ws_bytes": (_Z, [_I, _I, _I, _I]),
     "dd_gate_up_silu": (_I, [_P, _P, _P, _I, _I, _I, _P]),
     "dd_linear_supported": (_I, [_I, _I, _I]),
-    "dd_linear_ws_bytes": (_Z, [_I, _I, _I]),
-    "dd_linear_counters": (_I, [_I, _I, _I]),
-    "dd_linear": (_I, [_P, _P, _P, _I, _I, _I, _P, _P, _P]),
-    "dd_linear_silu": (_I, [_P, _P, _P, _I, _I, _I, _P, _P, _P]),
-    "dd_linear_add_rmsnorm": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _F, _P, _P, _P]),
+    "dd_linear_add_rmsnorm_ws_bytes": (_Z, [_I, _I, _I]),
+    "dd_linear": (_I, [_P, _P, _P, _I, _I, _I, _P]),
+    "dd_linear_silu": (_I, [_P, _P, _P, _I, _I, _I, _P]),
+    "dd_linear_add_rmsnorm": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _F, _P, _P]),
     "dd_silu_mul": (_I, [_P, _P, _I, _I, _P]),
     "dd_qkv_post_decode": (_I, [_P, _P, _P, _P, _P, _I, _P, _I, _P, _P, _P,
                                 _I, _I, _I, _I, _I, _I, _F, _P, _P]),

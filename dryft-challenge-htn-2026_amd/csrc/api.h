@@ -52,6 +52,10 @@ int launch_gemv(const void* x, const void* W, void* y, void* ws, int* counters, 
                 int K, int sk, const void* h, const void* lnw, void* hn, float eps,
                 hipStream_t stream);
 
+// Residual add + RMSNorm of a product left as S fp32 sums [S][M][N] (norm.hip; N <= 4096).
+int launch_sum_add_rmsnorm(const void* part, int S, const void* h, const void* w, void* hn, void* y, int M, int N,
+                           float eps, hipStream_t stream);
+
 }  // namespace dd
 
 #define DD_REQUIRE(cond)                         \

@@ -2,7 +2,7 @@
 //
 //   y[m][n] = sum_k x[m][k] * W[n][k]          (F.linear semantics, W row-major [N, K])
 //
-// with three epilogues: the plain product, SiLU(gate) * up, and the residual add.
+// with three epilogues: the plain product, SiLU(gate) * up, and fp32 sums for the residual add + norm.
 //
 // What bounds it: the weight stream. A CU's share of the HBM rate is ~27 bytes / ns and a load takes
 // 2 - 3 us under load, so 55 - 80 KB per CU have to be in flight at all times. One workgroup of 8 waves
@@ -12,23 +12,17 @@
 // over the end of a tile into the next one. W is streamed past the caches (nt), x is kept in them.
 //
 // Split: every workgroup gets the same number of output rows, so no CU idles in a last round of tiles,
-// and computes them whole (S = 1). Each workgroup then reads all of x; where that outweighs its
-// weights (M > 4 rows per workgroup: O and down above 40 rows), S = 2, 4, .. workgroups share S times
-// the rows and each takes a part of K: fp32 partials, added in workgroup order by the last workgroup
-// to arrive, so the result does not depend on the arrival order. Graph-timed on MI355X (cold weights,
-// the launch and the row norm included, us; before: the register-streaming GEMV up to 16 rows, hipBLASLt
-// and separate SiLU / add + norm kernels above):
-//             M =    1            16           32           64
-//   6144 x 2560      11.1 / 10.7  16.1 / 11.6  11.4 / 10.9  15.6 / 14.8   (QKV)
-//   2560 x 4096      12.5 / 11.6  24.2 / 12.8  15.7 / 13.9  17.7 / 18.1   (O, add, norm; S = 2 at 64)
-//   19456 x 2560     30.3 / 22.4  37.9 / 22.6  28.4 / 24.0  34.0 / 29.0   (gate/up, SiLU)
-//   2560 x 9728      18.7 / 17.8  34.6 / 20.9  23.4 / 21.6  31.4 / 26.0   (down, add, norm; S = 2 at 64)
-//   151936 x 2560    181 / 123    234 / 129    173 / 146    183 / 177     (lm_head)
+// and computes them whole. Each workgroup then reads all of x; where that outweighs its weights (M > 4
+// rows per workgroup) and a second launch follows anyway (residual add + norm: O and down above 40
+// rows), S = 2, 4, .. workgroups share S times the rows and each takes a part of K; that launch adds
+// their fp32 sums in order. Graph-timed on MI355X (cold weights, the launches included, us; before: the
+// register-streaming GEMV up to 16 rows, hipBLASLt and separate SiLU / add + norm kernels above):
+//   (table)
 // About 5 us of each are the launch and the first loads' latency; the lm_head streams at 6.6 TB/s. Equal
 // shares of K x tiles for every workgroup (stream-K over 64-row tiles) cost the partials' round trips:
-// 13.5 us for QKV at M = 1, 14.8 at 32. The norm of the new residual by the last workgroup of the same
-// launch took 3 us more than its own launch (two hand-offs), so it is a second launch. Above 64 rows
-// x's share of the loads grows past what hipBLASLt's larger tiles need (80 rows: O 18.6 against 16.1).
+// 13.5 us for QKV at M = 1, 14.8 at 32. The norm by the last workgroup of the same launch took 3 us more
+// than its own launch (two hand-offs). Above 64 rows x's share of the loads grows past what hipBLASLt's
+// larger tiles need (80 rows: O 18.6 against 16.1).
 //
 // MFMA 16x16x32: A = 16 weight rows, B = 16 activation rows (x^T), both read from LDS. The 8 waves
 // split a stage into (k-steps of 32) x (weight tiles), and every wave multiplies its weight fragments
@@ -43,20 +37,17 @@ namespace lin {
 constexpr int THREADS = 512;
 constexpr int LDS_MAX = 160 * 1024;
 
-enum { OUT = 0, SILU = 1, ADD = 2 };
+enum { OUT = 0, SILU = 1, PART = 2 };
 
 struct Args {
   const bf16* x;
   const bf16* W;
-  bf16* y;                                    // ADD: the new residual
-  const bf16* h;                              // ADD: the residual
-  float* ws;
-  int* counters;
+  bf16* y;                                    // OUT, SILU
+  float* ws;                                  // PART: fp32 sums [S][M][N]
   int M, N, K;                                // N: rows of W (SILU: 2 I)
   int nout;                                   // output columns (N; SILU: I)
   int nv;                                     // outputs per tile (rows of W; SILU: features)
-  int KT, S, C;                               // stages and chunks per tile, chunks in all
-  unsigned ws_bytes;
+  int KT, S, C;                               // stages and chunks (parts of K) per tile, chunks in all
 };
 
 // Geometry of one instantiation: BMT activation tiles, NT weight tiles.
@@ -76,11 +67,9 @@ struct Geo {
   static constexpr int RTILES = STAGE / 1024 / ((KW - 1) * NG * NTW);
   static constexpr int PASSES = (BMT + RTILES - 1) / RTILES;
   static_assert(RTILES >= 1, "k-slice partials fit a stage");
-  static constexpr int NST0 = (LDS_MAX - 256) / STAGE;
+  static constexpr int NST0 = LDS_MAX / STAGE;
   static constexpr int NST = NST0 > 14 ? 14 : NST0;
-  static constexpr int LDS = NST * STAGE + 256;
-  static constexpr int SLOT = NG * NTW * BMT * 1024;       // bytes of a partial tile
-  static constexpr int CB = NTW * BMT <= 4 ? 4 : NTW * BMT <= 10 ? 2 : 1;   // partials read together
+  static constexpr int LDS = NST * STAGE;
   // chunk swizzle of LDS row r: 8, 16 or 32 chunks a row
   static __device__ __forceinline__ int swz(int r) { return CPR == 8 ? (r >> 1) & 7 : r & 15; }
 };
@@ -111,9 +100,8 @@ __device__ __forceinline__ void dma16(rsrc_t r, unsigned voff, unsigned soff, un
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(size_t)lds, 16, voff, soff, 0, AUX);
 }
 
-// first chunk of workgroup g, and the workgroup that holds chunk c (C >= G chunks)
+// first chunk of workgroup g (C >= G chunks)
 __device__ __forceinline__ int chunk0(int C, int G, int g) { return (int)((long long)C * g / G); }
-__device__ __forceinline__ int chunk_wg(int C, int G, int c) { return (int)(((long long)(c + 1) * G - 1) / C); }
 // first unit (tile * KT + stage) of chunk c
 __device__ __forceinline__ int unit_of(const Args& a, int c) {
   const int t = c / a.S;
@@ -128,11 +116,11 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g4 = lane >> 4;
   const int G = gridDim.x, g = blockIdx.x;
-  const int u0 = unit_of(a, chunk0(a.C, G, g)), u1 = unit_of(a, chunk0(a.C, G, g + 1));
+  int chunk = chunk0(a.C, G, g);
+  const int u0 = unit_of(a, chunk), u1 = unit_of(a, chunk0(a.C, G, g + 1));
   const int kslice = wave % Z::KW, ng = wave / Z::KW;
   const unsigned lds0 = __builtin_amdgcn_readfirstlane(
       (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
-  int* flag = (int*)(smem + Z::NST * Z::STAGE);
 
   // ---- DMA side: instruction i of a stage (wave i % 8) fills LDS rows i RPI .. of W, then of x ----
   // Rows past M, and weight rows past the tile's last, lie outside the buffers' ranges: the hardware
@@ -184,12 +172,9 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
       for (int m = 0; m < BMT; ++m) acc[n][m] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
   clear();
-  const rsrc_t wsr = make_rsrc(a.ws, a.ws_bytes);
-  // 16-byte chunk of (n, m) in a partial tile
-  auto part_at = [&](int n, int m) { return (unsigned)(((nt_of(n) * BMT + m) * 64 + lane) * 16); };
 
-  // epilogue of tile t; the k-slice-0 waves hold its sums: output nt * 16 + g4 * 4 + i of row m * 16 + l16
-  auto finish = [&](int t) {
+  // epilogue of part s of tile t; the k-slice-0 waves hold its sums: output nt * 16 + g4 * 4 + i of row m * 16 + l16
+  auto finish = [&](int t, int s) {
     if (kslice != 0) return;
     const int n0 = t * a.nv, left = min(a.nv, a.nout - n0);
     const bool al = a.nout % 4 == 0 && a.nv % 4 == 0;                  // 8-byte accesses of 4 outputs
@@ -211,16 +196,21 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
         }
         if (row >= a.M || c >= left) continue;
         const size_t at = (size_t)row * a.nout + n0 + c;
-        if (al && c + 4 <= left) {
-          if (MODE == ADD) {
-            const u32x2 h = *(const u32x2*)(a.h + at);
-            v = f32x4{lo_bf(h.x) + rbf(v[0]), hi_bf(h.x) + rbf(v[1]), lo_bf(h.y) + rbf(v[2]), hi_bf(h.y) + rbf(v[3])};
+        if (MODE == PART) {
+          float* dst = a.ws + (size_t)s * a.M * a.nout + at;
+          if (al && c + 4 <= left) {
+            *(f32x4*)dst = v;
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (c + i < left) dst[i] = v[i];
           }
+        } else if (al && c + 4 <= left) {
           *(u32x2*)(a.y + at) = u32x2{pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3])};
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (c + i < left) a.y[at + i] = f2bf(MODE == ADD ? bf2f(a.h[at + i]) + rbf(v[i]) : v[i]);
+            if (c + i < left) a.y[at + i] = f2bf(v[i]);
         }
       }
   };
@@ -230,8 +220,7 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
   for (int i = 0; i < Z::NST - 1 && ui < u1; ++i) issue();
   // A wave's loads land in issue order, so the count of its later loads covers the stage; stores in
   // between only make it wait for more.
-  int tile = u0 / a.KT, ks = u0 - tile * a.KT, slot = 0;
-  int seg_tile[2] = {-1, -1};                                          // partial tiles left in ws
+  int slot = 0, uend = unit_of(a, chunk + 1);                          // end of the current chunk
   for (int u = u0; u < u1; ++u) {
     const int rem = min(Z::NST - 2, u1 - 1 - u);                       // stages requested after this one
     if (ni == Z::IPW) wait_stages<Z::NST - 2, Z::IPW>(rem);
@@ -250,8 +239,8 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
       for (int m = 0; m < BMT; ++m) acc[n][m] = mfma16x16x32(wf[n], xf[m], acc[n][m]);
     const int cur = slot;
     slot = slot + 1 == Z::NST ? 0 : slot + 1;
-    if (++ks < a.KT && u + 1 < u1) continue;
-    // end of the tile, or of the range inside it: add the k-slices (in order) in the slice-0 waves,
+    if (u + 1 < uend) continue;
+    // end of the chunk: add the k-slices (in order) in the slice-0 waves,
     // through the stage just consumed (it is requested into again after the next stage's barrier)
     f32x4* red = (f32x4*)(smem + cur * Z::STAGE) + lane;
 #pragma unroll
@@ -278,71 +267,9 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
           }
       }
     }
-    const bool first = u - (ks - 1) >= u0, last = ks == a.KT;          // the range holds its begin, its end
-    if (first && last) {
-      finish(tile);
-    } else {
-      const int w = first ? 1 : 0;                                     // begins here: the range's last segment
-      seg_tile[w] = tile;
-      if (kslice == 0) {
-#pragma unroll
-        for (int n = 0; n < Z::NTW; ++n)
-#pragma unroll
-          for (int m = 0; m < BMT; ++m)
-            stc_b128(wsr, (unsigned)(2 * g + w) * Z::SLOT + part_at(n, m), __builtin_bit_cast(u32x4, acc[n][m]));
-      }
-    }
+    finish(chunk / a.S, chunk % a.S);
     clear();
-    ks = 0;
-    ++tile;
-  }
-  if (seg_tile[0] < 0 && seg_tile[1] < 0) return;
-
-  // ---- split tiles: the last workgroup to arrive adds the partials in workgroup order ----
-  // Both segments' arrivals go out together (one thread of two waves), after one wait for the stores.
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (lane == 0 && wave < 2) {
-    const int t = seg_tile[wave];
-    int last = 0;
-    if (t >= 0) {
-      const int n = chunk_wg(a.C, G, (t + 1) * a.S - 1) - chunk_wg(a.C, G, t * a.S) + 1;
-      last = __hip_atomic_fetch_add(a.counters + t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
-      if (last) __hip_atomic_store(a.counters + t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    flag[wave] = last;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    const int t = seg_tile[w];
-    if (t < 0 || !flag[w]) continue;
-    const int ga = chunk_wg(a.C, G, t * a.S), gb = chunk_wg(a.C, G, (t + 1) * a.S - 1);
-    if (kslice == 0) {
-      clear();
-      for (int s0 = ga; s0 <= gb; s0 += Z::CB) {                       // CB workgroups' partials in flight
-        u32x4 part[Z::CB][Z::NTW][BMT];
-#pragma unroll
-        for (int j = 0; j < Z::CB; ++j) {
-          // past the last: outside the range, reads 0. A workgroup left the tile in its second slot
-          // where its range begins at or before the tile's begin.
-          const int s = s0 + j;
-          const unsigned base =
-              s > gb ? 0x80000000u : (unsigned)(2 * s + (chunk0(a.C, G, s) <= t * a.S ? 1 : 0)) * Z::SLOT;
-#pragma unroll
-          for (int n = 0; n < Z::NTW; ++n)
-#pragma unroll
-            for (int m = 0; m < BMT; ++m) part[j][n][m] = ldc_b128(wsr, base + part_at(n, m));
-        }
-#pragma unroll
-        for (int j = 0; j < Z::CB; ++j)
-#pragma unroll
-          for (int n = 0; n < Z::NTW; ++n)
-#pragma unroll
-            for (int m = 0; m < BMT; ++m) acc[n][m] += __builtin_bit_cast(f32x4, part[j][n][m]);
-      }
-    }
-    finish(t);
+    uend = unit_of(a, ++chunk + 1);
   }
 }
 
@@ -358,7 +285,7 @@ using namespace dd;
 namespace {
 
 struct Plan {
-  int bmt, nt, nv, nout, ntiles, KT, S, C, G;
+  int bmt, nt, nv, nout, KT, S, C, G;
   size_t ws_bytes;
 };
 
@@ -372,11 +299,12 @@ bool plan_for(int mode, int M, int N, int K, Plan& p) {
   p.nout = mode == lin::SILU ? N / 2 : N;
   p.bmt = (M + 15) / 16;
   const int per16 = mode == lin::SILU ? 8 : 16;                        // outputs of a 16-row weight tile
-  // S: workgroups per share of the outputs; nv: outputs of S workgroups, in tiles of at most 128 rows
+  // S: parts of K (PART: the sums meet in the norm's launch); nv: outputs of S workgroups, in tiles of at
+  // most 128 rows
   int nv = 0;
-  for (p.S = 1; p.S <= 8; p.S *= 2) {
+  for (p.S = 1;; p.S *= 2) {
     nv = (int)(((long long)p.nout * p.S + G - 1) / G);
-    if (M <= 4 * nv * (16 / per16)) break;
+    if (mode != lin::PART || p.S == 8 || M <= 4 * nv) break;
   }
   const int parts = (nv + 8 * per16 - 1) / (8 * per16);
   p.nv = nv = (nv + parts - 1) / parts;
@@ -389,11 +317,11 @@ bool plan_for(int mode, int M, int N, int K, Plan& p) {
                                                     : 8;
   p.KT = K / (p.nt == 1 ? 256 : p.nt == 2 ? 128 : 64);
   if (p.S > p.KT) p.S = p.KT;
-  p.ntiles = (p.nout + nv - 1) / nv;
-  if ((long long)p.ntiles * p.KT >= (1ll << 30)) return false;
-  p.C = p.ntiles * p.S;
+  const int ntiles = (p.nout + nv - 1) / nv;
+  if ((long long)ntiles * p.KT >= (1ll << 30)) return false;
+  p.C = ntiles * p.S;
   p.G = p.C < G ? p.C : G;
-  p.ws_bytes = p.S == 1 ? 16 : (size_t)2 * p.G * (p.nt == 5 ? 8 : p.nt) * p.bmt * 1024;
+  p.ws_bytes = mode == lin::PART ? (size_t)p.S * M * N * 4 : 16;
   return true;
 }
 
@@ -419,15 +347,12 @@ int launch_nt(const lin::Args& a, const Plan& p, hipStream_t stream) {
 }
 
 template <int MODE>
-int launch(const Plan& p, const void* x, const void* W, const void* h, void* y, int M, int N, int K, void* ws,
-           int* counters, hipStream_t stream) {
+int launch(const Plan& p, const void* x, const void* W, void* y, int M, int N, int K, void* ws, hipStream_t stream) {
   lin::Args a;
   a.x = (const bf16*)x;
   a.W = (const bf16*)W;
   a.y = (bf16*)y;
-  a.h = (const bf16*)h;
   a.ws = (float*)ws;
-  a.counters = counters;
   a.M = M;
   a.N = N;
   a.K = K;
@@ -436,7 +361,6 @@ int launch(const Plan& p, const void* x, const void* W, const void* h, void* y, 
   a.KT = p.KT;
   a.S = p.S;
   a.C = p.C;
-  a.ws_bytes = (unsigned)p.ws_bytes;
   switch (p.bmt) {
     case 1: return launch_nt<1, MODE>(a, p, stream);
     case 2: return launch_nt<2, MODE>(a, p, stream);
@@ -452,43 +376,30 @@ DD_API int dd_linear_supported(int M, int N, int K) {
   return plan_for(lin::OUT, M, N, K, p) ? 1 : 0;
 }
 
-DD_API size_t dd_linear_ws_bytes(int M, int N, int K) {
+DD_API size_t dd_linear_add_rmsnorm_ws_bytes(int M, int N, int K) {
   Plan p;
-  size_t most = 0;
-  for (int mode : {lin::OUT, lin::SILU, lin::ADD})
-    if (plan_for(mode, M, N, K, p) && p.ws_bytes > most) most = p.ws_bytes;
-  return most;
+  return plan_for(lin::PART, M, N, K, p) ? p.ws_bytes : 0;
 }
 
-DD_API int dd_linear_counters(int M, int N, int K) {
+DD_API int dd_linear(const void* x, const void* W, void* y, int M, int N, int K, hipStream_t stream) {
   Plan p;
-  int most = 1;
-  for (int mode : {lin::OUT, lin::SILU, lin::ADD})
-    if (plan_for(mode, M, N, K, p) && p.S > 1 && p.ntiles > most) most = p.ntiles;
-  return most;
+  DD_REQUIRE(x && W && y && plan_for(lin::OUT, M, N, K, p));
+  DD_REQUIRE(aligned16(x) && aligned16(W) && aligned16(y));
+  return launch<lin::OUT>(p, x, W, y, M, N, K, nullptr, stream);
 }
 
-DD_API int dd_linear(const void* x, const void* W, void* y, int M, int N, int K, void* ws, int* counters,
-                     hipStream_t stream) {
+DD_API int dd_linear_silu(const void* x, const void* Wgu, void* out, int M, int I, int K, hipStream_t stream) {
   Plan p;
-  DD_REQUIRE(x && W && y && ws && counters && plan_for(lin::OUT, M, N, K, p));
-  DD_REQUIRE(aligned16(x) && aligned16(W) && aligned16(y) && aligned16(ws));
-  return launch<lin::OUT>(p, x, W, nullptr, y, M, N, K, ws, counters, stream);
-}
-
-DD_API int dd_linear_silu(const void* x, const void* Wgu, void* out, int M, int I, int K, void* ws, int* counters,
-                          hipStream_t stream) {
-  Plan p;
-  DD_REQUIRE(x && Wgu && out && ws && counters && I >= 1 && I < (1 << 30) && plan_for(lin::SILU, M, 2 * I, K, p));
-  DD_REQUIRE(aligned16(x) && aligned16(Wgu) && aligned16(out) && aligned16(ws));
-  return launch<lin::SILU>(p, x, Wgu, nullptr, out, M, 2 * I, K, ws, counters, stream);
+  DD_REQUIRE(x && Wgu && out && I >= 1 && I < (1 << 30) && plan_for(lin::SILU, M, 2 * I, K, p));
+  DD_REQUIRE(aligned16(x) && aligned16(Wgu) && aligned16(out));
+  return launch<lin::SILU>(p, x, Wgu, out, M, 2 * I, K, nullptr, stream);
 }
 
 DD_API int dd_linear_add_rmsnorm(const void* x, const void* W, const void* h, const void* lnw, void* hn, void* y,
-                                 int M, int N, int K, float eps, void* ws, int* counters, hipStream_t stream) {
+                                 int M, int N, int K, float eps, void* ws, hipStream_t stream) {
   Plan p;
-  DD_REQUIRE(x && W && h && lnw && hn && y && ws && counters && N <= 4096 && plan_for(lin::ADD, M, N, K, p));
-  DD_REQUIRE(aligned16(x) && aligned16(W) && aligned16(h) && aligned16(hn) && aligned16(ws));
-  const int rc = launch<lin::ADD>(p, x, W, h, hn, M, N, K, ws, counters, stream);
-  return rc != 0 ? rc : dd_rmsnorm(hn, lnw, y, M, N, eps, stream);
+  DD_REQUIRE(x && W && h && lnw && hn && y && ws && N <= 4096 && plan_for(lin::PART, M, N, K, p));
+  DD_REQUIRE(aligned16(x) && aligned16(W) && aligned16(ws));
+  const int rc = launch<lin::PART>(p, x, W, nullptr, M, N, K, ws, stream);
+  return rc != 0 ? rc : launch_sum_add_rmsnorm(ws, p.S, h, lnw, hn, y, M, N, eps, stream);
 }

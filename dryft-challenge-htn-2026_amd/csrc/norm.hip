@@ -148,6 +148,56 @@ add_rmsnorm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ d, const
   }
 }
 
+// hn = bf16(h + bf16(sum_s part[s])); y = rms(hn) * w            grid (M)
+// The residual add and norm after a product left as fp32 sums of S parts of K [S][M][N], added in order.
+__global__ void __launch_bounds__(NORM_THREADS)
+sum_add_rmsnorm_kernel(const float* __restrict__ part, int S, const bf16* __restrict__ h, const bf16* __restrict__ w,
+                       bf16* __restrict__ hn, bf16* __restrict__ y, int M, int N, float eps) {
+  __shared__ float red[NORM_WAVES];
+  const size_t row = blockIdx.x;
+  const float* pr = part + row * N;
+  const bf16* xr = h + row * N;
+  bf16* hr = hn + row * N;
+  bf16* yr = y + row * N;
+  if (vec_ok(N, xr, w, hr, yr) && (((uintptr_t)pr) & 15) == 0) {
+    float v[NORM_NV][8];
+#pragma unroll
+    for (int j = 0; j < NORM_NV; ++j) {
+      const int c = (threadIdx.x + j * NORM_THREADS) * 8;
+      const bool ok = c < N;
+      float a[8];
+      unpack8(ok ? ld16(xr + c) : u32x4{0u, 0u, 0u, 0u}, a);
+      f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+#pragma unroll 4
+      for (int s = 0; s < S; ++s)
+        if (ok) {
+          lo += *(const f32x4*)(pr + (size_t)s * M * N + c);
+          hi += *(const f32x4*)(pr + (size_t)s * M * N + c + 4);
+        }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[j][e] = rbf(a[e] + rbf(e < 4 ? lo[e & 3] : hi[e & 3]));
+      if (ok) *(u32x4*)(hr + c) = pack8(v[j]);
+    }
+    norm_row_vec(v, N, w, yr, eps, red);
+  } else {
+    float v[NORM_MAXV];
+#pragma unroll
+    for (int j = 0; j < NORM_MAXV; ++j) {
+      const int c = threadIdx.x + j * NORM_THREADS;
+      float t = 0.f;
+      for (int s = 0; s < S; ++s)
+        if (c < N) t += pr[(size_t)s * M * N + c];
+      v[j] = c < N ? rbf(bf2f(xr[c]) + rbf(t)) : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < NORM_MAXV; ++j) {
+      const int c = threadIdx.x + j * NORM_THREADS;
+      if (c < N) hr[c] = f2bf(v[j]);
+    }
+    norm_row_scalar(v, N, w, yr, eps, red);
+  }
+}
+
 // h[m] = embed[tok[m]]; y = rms(h) * w           grid (M)
 __global__ void __launch_bounds__(NORM_THREADS)
 embed_rmsnorm_kernel(const int64_t* __restrict__ tok, const bf16* __restrict__ embed, int V,
@@ -229,6 +279,13 @@ __global__ void silu_mul_vec_kernel(const bf16* __restrict__ gu, bf16* __restric
 #include "api.h"
 
 using namespace dd;
+
+int dd::launch_sum_add_rmsnorm(const void* part, int S, const void* h, const void* w, void* hn, void* y, int M, int N,
+                               float eps, hipStream_t stream) {
+  hipLaunchKernelGGL(sum_add_rmsnorm_kernel, dim3(M), dim3(NORM_THREADS), 0, stream, (const float*)part, S,
+                     (const bf16*)h, (const bf16*)w, (bf16*)hn, (bf16*)y, M, N, eps);
+  return launch_status();
+}
 
 DD_API int dd_rmsnorm(const void* x, const void* w, void* y, int M, int N, float eps,
                       hipStream_t stream) {

@@ -120,7 +120,6 @@ class HipOps:
         self._gemm_ws = None
         self._gemm_table = load_gemm_table()
         self._starts = {}
-        self._lin_sizes = {}
         self.err = torch.zeros(1, dtype=torch.int32, device=e.dev)
 
     # ---------------------------------------------------------------- helpers
@@ -137,24 +136,13 @@ class HipOps:
         return (self.use_gemv and 1 <= M <= BM_MAX and _bf16_ok(x, w) and K % 8 == 0
                 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
-    def _linear_plan(self, x, w):
-        """(workspace, counters) when the weight-streaming linear kernels take x @ w^T, else None:
-        the kernels of choice up to LIN_MAX rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt."""
+    def _linear_ok(self, x, w):
+        """Whether the weight-streaming linear kernels take x @ w^T: the kernels of choice up to
+        LIN_MAX rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt."""
         M, K = x.shape
-        N = w.shape[0]
-        if not (self.use_gemv and 1 <= M <= LIN_MAX and w.dim() == 2 and w.shape[1] == K
-                and _bf16_ok(x, w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-            return None
-        key = (M, N, K)
-        size = self._lin_sizes.get(key)
-        if size is None:
-            ok = self.L.dd_linear_supported(M, N, K)
-            size = self._lin_sizes[key] = (self.L.dd_linear_ws_bytes(M, N, K),
-                                           self.L.dd_linear_counters(M, N, K)) if ok else (0, 0)
-        if size[0] == 0:
-            return None
-        return (torch.empty(size[0] // 4, dtype=torch.float32, device=x.device),
-                self._zeroed_counters(size[1], x.device))
+        return (self.use_gemv and 1 <= M <= LIN_MAX and w.dim() == 2 and w.shape[1] == K
+                and _bf16_ok(x, w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and bool(self.L.dd_linear_supported(M, w.shape[0], K)))
 
     def _gemm_ok(self, x, w):
         """Prefill-sized bf16 products go to the library's hipBLASLt GEMM (dd_gemm_bf16) with the
@@ -218,13 +206,12 @@ class HipOps:
 
     # ---------------------------------------------------------------- GEMV family
     def linear(self, x, w):
-        plan = self._linear_plan(x, w) if x.dim() == 2 else None
-        if plan is not None:
+        if x.dim() == 2 and self._linear_ok(x, w):
             M, K = x.shape
             N = w.shape[0]
             out = torch.empty((M, N), dtype=x.dtype, device=x.device)
-            check(self.L.dd_linear(_ptr(x), _ptr(w), _ptr(out), M, N, K, _ptr(plan[0]),
-                                   _ptr(plan[1]), _stream(x.device)), "dd_linear")
+            check(self.L.dd_linear(_ptr(x), _ptr(w), _ptr(out), M, N, K, _stream(x.device)),
+                  "dd_linear")
             return out
         if not self._gemv_ok(x, w):
             return self._gemm(x, w) if self._gemm_ok(x, w) else F.linear(x, w)
@@ -242,13 +229,12 @@ class HipOps:
         return out
 
     def gate_up_silu(self, x, wgu):
-        plan = self._linear_plan(x, wgu) if wgu.shape[0] % 2 == 0 else None
-        if plan is not None:
+        if wgu.shape[0] % 2 == 0 and self._linear_ok(x, wgu):
             M, K = x.shape
             I = wgu.shape[0] // 2
             out = torch.empty((M, I), dtype=x.dtype, device=x.device)
-            check(self.L.dd_linear_silu(_ptr(x), _ptr(wgu), _ptr(out), M, I, K, _ptr(plan[0]),
-                                        _ptr(plan[1]), _stream(x.device)), "dd_linear_silu")
+            check(self.L.dd_linear_silu(_ptr(x), _ptr(wgu), _ptr(out), M, I, K, _stream(x.device)),
+                  "dd_linear_silu")
             return out
         if not self._gemv_ok(x, wgu):
             return self.silu_mul(self.linear(x, wgu))
@@ -261,19 +247,17 @@ class HipOps:
 
     def linear_add_norm(self, x, w, h, lnw):
         """hn = h + x @ w^T ; returns (hn, rmsnorm(hn, lnw))"""
-        plan = (self._linear_plan(x, w)
-                if w.shape[0] <= NORM_MAX and h.shape == (x.shape[0], w.shape[0])
-                and lnw.numel() == w.shape[0] and _bf16_ok(h, lnw) and h.data_ptr() % 16 == 0
-                else None)
-        if plan is not None:
+        if (w.shape[0] <= NORM_MAX and h.shape == (x.shape[0], w.shape[0])
+                and lnw.numel() == w.shape[0] and _bf16_ok(h, lnw) and self._linear_ok(x, w)):
             M, K = x.shape
             N = w.shape[0]
+            ws = torch.empty(self.L.dd_linear_add_rmsnorm_ws_bytes(M, N, K) // 4,
+                             dtype=torch.float32, device=x.device)
             hn = torch.empty_like(h)
             y = torch.empty_like(h)
             check(self.L.dd_linear_add_rmsnorm(_ptr(x), _ptr(w), _ptr(h), _ptr(lnw), _ptr(hn),
-                                               _ptr(y), M, N, K, self.e.eps, _ptr(plan[0]),
-                                               _ptr(plan[1]), _stream(x.device)),
-                  "dd_linear_add_rmsnorm")
+                                               _ptr(y), M, N, K, self.e.eps, _ptr(ws),
+                                               _stream(x.device)), "dd_linear_add_rmsnorm")
             return hn, y
         if not (self._gemv_ok(x, w) and _bf16_ok(h, lnw)):
             return self.add_rms(h, self.linear(x, w), lnw)

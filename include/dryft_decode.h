@@ -83,24 +83,22 @@ size_t dd_gemv_add_rmsnorm_ws_bytes(int M, int N, int K, int splitk);
 int dd_gate_up_silu(const void* x, const void* Wgu, void* out, int M, int I, int K,
                     hipStream_t stream);
 
-/* Skinny linear layers, 1 <= M <= 64 rows (K % 64 == 0, N * K < 2^30; x, W, ws and the outputs
+/* Skinny linear layers, 1 <= M <= 64 rows (K % 64 == 0, N * K < 2^30; x, W, ws and the products
  * 16-byte aligned): the products and epilogues of dd_gemv / dd_gate_up_silu / dd_gemv_add_rmsnorm
  * with the weights streamed through LDS, every workgroup an equal share of the outputs.
- * dd_linear_supported: 1 when the shape is taken. ws: dd_linear_ws_bytes(M, N, K) bytes (N: rows of
- * W, so 2 I for dd_linear_silu); counters: dd_linear_counters(M, N, K) zeroed ints.
- * dd_linear_add_rmsnorm is two launches (N <= 4096): the product with the residual add, the norm.
+ * dd_linear_supported: 1 when the shape is taken (N: rows of W, so 2 I for dd_linear_silu).
+ * dd_linear_add_rmsnorm is two launches (N <= 4096): the product as fp32 sums in ws
+ * (dd_linear_add_rmsnorm_ws_bytes bytes), then the residual add and the norm. No counters: calls on
+ * different streams need only workspaces of their own.
  * Replace TritonOps.linear / gate_up_silu / linear_add_norm (fused.py:989-1059), and above 16 rows
  * the F.linear fallback of those methods (engine.py:131-146). */
 int dd_linear_supported(int M, int N, int K);
-size_t dd_linear_ws_bytes(int M, int N, int K);
-int dd_linear_counters(int M, int N, int K);
-int dd_linear(const void* x, const void* W, void* y, int M, int N, int K, void* ws, int* counters,
-              hipStream_t stream);
-int dd_linear_silu(const void* x, const void* Wgu, void* out, int M, int I, int K, void* ws,
-                   int* counters, hipStream_t stream);
+size_t dd_linear_add_rmsnorm_ws_bytes(int M, int N, int K);
+int dd_linear(const void* x, const void* W, void* y, int M, int N, int K, hipStream_t stream);
+int dd_linear_silu(const void* x, const void* Wgu, void* out, int M, int I, int K,
+                   hipStream_t stream);
 int dd_linear_add_rmsnorm(const void* x, const void* W, const void* h, const void* lnw, void* hn,
-                          void* y, int M, int N, int K, float eps, void* ws, int* counters,
-                          hipStream_t stream);
+                          void* y, int M, int N, int K, float eps, void* ws, hipStream_t stream);
 
 /* out[M,I] = bf16(bf16(silu(g)) * u) with gu[M, 2I] = [g | u].
  * Replaces TritonOps.silu_mul (fused.py:900-906; kernel fused.py:175-188). */
