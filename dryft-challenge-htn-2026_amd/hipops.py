@@ -30,6 +30,7 @@ NORM_MAX = 4096  # longest row the row-norm kernels take
 # Smallest row count sent to the library's own hipBLASLt call: everything past the skinny kernels.
 # (F.linear asks hipBLASLt's heuristic again on every call, 21 us of host time against 6.)
 GEMM_MIN_M = LIN_MAX + 1
+GEMM_WS_MAX = 8  # hipBLASLt workspaces an ops object keeps (64 MiB each)
 
 
 def _ptr(t):
@@ -71,6 +72,11 @@ def _stream(dev):
     object around it: 4.5 us a launch, a third of a small launch's host time)."""
     i = dev.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
+
+
+def _wants_grad(*ts):
+    """Whether autograd would record an op on these: F.linear is differentiable, the kernels are not."""
+    return torch.is_grad_enabled() and any(t.requires_grad for t in ts)
 
 
 def _bf16_ok(*ts):
@@ -117,7 +123,7 @@ class HipOps:
         assert e.hd & (e.hd - 1) == 0 and e.hd >= 2
         self.L = lib()  # raises when the library is missing: no silent fallback
         self._counters = None
-        self._gemm_ws = None
+        self._gemm_ws = {}  # hipBLASLt workspaces by (device, stream), at most GEMM_WS_MAX
         self._gemm_table = load_gemm_table()
         self._starts = {}
         self.err = torch.zeros(1, dtype=torch.int32, device=e.dev)
@@ -138,17 +144,22 @@ class HipOps:
 
     def _linear_ok(self, x, w):
         """Whether the weight-streaming linear kernels take x @ w^T: the kernels of choice up to
-        LIN_MAX rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt."""
+        LIN_MAX rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt. Operands that need a
+        gradient keep F.linear above the GEMV's rows."""
         M, K = x.shape
         return (self.use_gemv and 1 <= M <= LIN_MAX and w.dim() == 2 and w.shape[1] == K
+                and (M <= BM_MAX or not _wants_grad(x, w))
                 and _bf16_ok(x, w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
                 and bool(self.L.dd_linear_supported(M, w.shape[0], K)))
 
     def _gemm_ok(self, x, w):
         """Prefill-sized bf16 products go to the library's hipBLASLt GEMM (dd_gemm_bf16) with the
-        solution the committed table names for the shape; DD_TUNED_GEMM=0 keeps them on F.linear
-        (diagnostics)."""
-        return (x.dim() == 2 and x.shape[0] >= GEMM_MIN_M and _bf16_ok(x, w)
+        solution the committed table names for the shape. F.linear keeps what the call cannot take
+        (it raises for mismatched shapes): other ranks, unaligned operands, operands that need a
+        gradient. DD_TUNED_GEMM=0 keeps all of them there (diagnostics)."""
+        return (x.dim() == w.dim() == 2 and x.shape[0] >= GEMM_MIN_M and x.shape[1] == w.shape[1]
+                and w.shape[0] > 0 and x.shape[1] > 0 and _bf16_ok(x, w) and x.device == w.device
+                and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not _wants_grad(x, w)
                 and os.environ.get("DD_TUNED_GEMM", "1") != "0")
 
     def _gemm_lib(self, x, w, solution=None):
@@ -156,14 +167,25 @@ class HipOps:
         N = w.shape[0]
         if solution is None:
             solution = gemm_solution(self._gemm_table, N, K, M)
-        ws = self._gemm_ws
-        if ws is None or ws.device != x.device:
-            ws = self._gemm_ws = torch.empty(self.L.dd_gemm_ws_bytes(), dtype=torch.uint8,
-                                             device=x.device)
+        stream = _stream(x.device)
+        ws = self._gemm_workspace(x.device, stream)
         y = torch.empty((M, N), dtype=x.dtype, device=x.device)
         check(self.L.dd_gemm_bf16(_ptr(x), _ptr(w), _ptr(y), M, N, K, _ptr(ws), ws.numel(),
-                                  solution, _stream(x.device)), "dd_gemm_bf16")
+                                  solution, stream), "dd_gemm_bf16")
         return y
+
+    def _gemm_workspace(self, dev, stream):
+        """hipBLASLt's workspace for a product on `stream`: kept per stream, since products on two
+        streams would write the same one; a captured product gets one of its graph's own pool."""
+        if torch.cuda.is_current_stream_capturing():
+            return torch.empty(self.L.dd_gemm_ws_bytes(), dtype=torch.uint8, device=dev)
+        ws = self._gemm_ws.get((dev, stream))
+        if ws is None:
+            if len(self._gemm_ws) >= GEMM_WS_MAX:
+                self._gemm_ws.clear()  # each goes back to the allocator, in its own stream's order
+            ws = self._gemm_ws[dev, stream] = torch.empty(self.L.dd_gemm_ws_bytes(),
+                                                          dtype=torch.uint8, device=dev)
+        return ws
 
     def _gemm(self, x, w):
         """y = x . w^T on hipBLASLt with the table's solution for (N, K, M): a fixed choice per

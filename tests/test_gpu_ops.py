@@ -226,6 +226,35 @@ def test_linear_add_norm_real(small, weights, name):
         close(y, ry)
 
 
+@pytest.mark.parametrize("M", [17, 64, 65, 300])
+def test_linear_keeps_what_only_f_linear_takes(small, M):
+    """Products above the GEMV's rows: mismatched shapes raise, an operand that needs a gradient gets it,
+    an unaligned operand goes to F.linear, and products on two streams do not share a workspace."""
+    hip = small[1]
+    g = torch.Generator().manual_seed(M)
+    x = torch.randint(-1, 2, (M, 192), generator=g).to(BF).cuda()
+    w = torch.randint(-1, 2, (80, 192), generator=g).to(BF).cuda()
+    ref = x.float() @ w.float().t()
+    with pytest.raises(RuntimeError):
+        hip.linear(x, w[:, :128].contiguous())
+    wg = w.clone().requires_grad_()
+    y = hip.linear(x, wg)
+    assert torch.equal(y.float(), ref)
+    y.backward(torch.ones_like(y))
+    assert torch.equal(wg.grad[0].float(), x.float().sum(0).to(BF).float())
+    odd = torch.empty(M * 192 + 1, dtype=BF, device="cuda")[1:].view(M, 192).copy_(x)
+    assert odd.data_ptr() % 16 != 0 and not hip._linear_ok(odd, w) and not hip._gemm_ok(odd, w)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        z = hip.linear(x, w)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(z.float(), ref) and torch.equal(hip.linear(x, w).float(), ref)
+    if M > 64:
+        a, b = (hip._gemm_workspace(x.device, s.cuda_stream) for s in (side, torch.cuda.current_stream()))
+        assert a.data_ptr() != b.data_ptr()
+
+
 # rows at the edges of the 16-row tiles; N and K at a ragged last tile, tiles of 1 / 2 / 4 / 5 / 8 weight
 # tiles, K split over workgroups (few outputs, many rows) and every stage width
 @pytest.mark.parametrize("M", [1, 16, 17, 48, 64])
