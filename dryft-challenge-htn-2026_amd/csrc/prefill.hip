@@ -400,8 +400,8 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
   bf16* const shk = (bf16*)pp_smem;
   bf16* const shv = shk + NB * BUF;
   int b = 0, p0 = 0;
-  if (!tile_of(seq_start, B, blockIdx.y, last_only != 0, TQ, b, p0)) return;
-  const int kvh = blockIdx.x;
+  const int tile = blockIdx.x / NKV, kvh = blockIdx.x - tile * NKV;   // one dimension: a grid's y ends at 65,535
+  if (!tile_of(seq_start, B, tile, last_only != 0, TQ, b, p0)) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l32 = lane & 31, h = lane >> 5;
   const bool late = wave >= 4;                                  // one phase behind (waves w, w + 4 share a SIMD)
@@ -423,7 +423,7 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
   // DMA: instruction i fills rows 4 i .. 4 i + 3 of a buffer; wave w issues IPW of them. Rows past the
   // prompt repeat its last key (masked); blocks past the last repeat it (not used).
   auto dma = [&](rsrc_t r, unsigned voff, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds) : "m0", "memory");
   };
   const int drow = 4 * IPW * wave + (lane >> 4), dc = lane & 15;
   auto issue_k = [&](int j, int buf) {
@@ -688,7 +688,7 @@ DD_API int dd_attn_prefill(const void* q, const void* kc, const void* vc, const 
     attr = allow_lds((const void*)kern, pf::pp_lds(nw), nw == 8 ? done8 : done4);
     if (attr != hipSuccess) return;
     const int ntiles = last_only ? B : T / (8 * nw) + B;
-    hipLaunchKernelGGL(kern, dim3(NKV, ntiles), dim3(64 * nw), pf::pp_lds(nw), stream, (const bf16*)q, (const bf16*)kc,
+    hipLaunchKernelGGL(kern, dim3((unsigned)ntiles * NKV), dim3(64 * nw), pf::pp_lds(nw), stream, (const bf16*)q, (const bf16*)kc,
                        (const bf16*)vc, seq_start, B, T, (bf16*)out, NH, NKV, cap, last_only, scale_log2);
   };
   switch (G) {

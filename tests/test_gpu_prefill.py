@@ -171,9 +171,8 @@ def test_attn_prefill_packed(cuda, lens, NH, NKV, cap):
 
 
 def test_attn_prefill_dma_equals_register_staging(cuda):
-    """G = 4 runs the LDS-DMA kernel when the cache capacity is a multiple of 32 and the
-    register-staged kernel otherwise; both compute the same arithmetic, so the same prompts in a
-    cache of 256 and of 264 slots give identical bits (and the fp64 bound holds for both)."""
+    """The cache's capacity (here a multiple of the key block and not) does not change a bit: the same
+    prompts in a cache of 256 and of 264 slots give identical results (and the fp64 bound holds)."""
     lens, NH, NKV = (1, 31, 32, 33, 200, 256), 32, 8
     B = len(lens)
     hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
@@ -196,6 +195,17 @@ def test_attn_prefill_dma_equals_register_staging(cuda):
     for k, v in ((kc, vc), (kc2, vc2)):
         ol = hip.attn_prefill_packed(qg[last].contiguous(), k.cuda(), v.cuda(), ss, B, T, last_only=True)
         assert torch.equal(ol, dma[last.cuda()])
+
+
+def test_attn_prefill_more_prompts_than_a_grid_dimension(cuda):
+    """65,600 prompts of one token (a grid's second dimension ends at 65,535): each row is its own value."""
+    hip = _hip(fake_engine(nh=4, nkv=1, hd=HD, rope_len=16))
+    B = 65600
+    q = torch.randn(B, 4, HD, device="cuda").to(BF)
+    kc, vc = (torch.randn(B, 1, 1, HD, device="cuda").to(BF) for _ in range(2))
+    start = torch.arange(B + 1, dtype=torch.int32, device="cuda")
+    out = hip.attn_prefill_packed(q, kc, vc, start, B, B, last_only=True)
+    assert torch.equal(out.view(B, 4, HD), vc.view(B, 1, HD).expand(B, 4, HD))
 
 
 def test_attn_prefill_through_reference_interface(cuda):
