@@ -1,4 +1,5 @@
-// Skinny linear layers (1 <= M <= 64 activation rows) that stream the weights through LDS, gfx950.
+// Skinny linear layers (1 <= M <= 64 activation rows; with the SiLU epilogue up to 96, with the sums up to
+// 128) that stream the weights through LDS, gfx950.
 //
 //   y[m][n] = sum_k x[m][k] * W[n][k]          (F.linear semantics, W row-major [N, K])
 //
@@ -15,14 +16,29 @@
 // and computes them whole. Each workgroup then reads all of x; where that outweighs its weights (M > 4
 // rows per workgroup) and a second launch follows anyway (residual add + norm: O and down above 40
 // rows), S = 2, 4, .. workgroups share S times the rows and each takes a part of K; that launch adds
-// their fp32 sums in order. Graph-timed on MI355X (cold weights, the launches included, us; before: the
-// register-streaming GEMV up to 16 rows, hipBLASLt and separate SiLU / add + norm kernels above):
-//   (table)
-// About 5 us of each are the launch and the first loads' latency; the lm_head streams at 6.6 TB/s. Equal
+// their fp32 sums in order. Graph-timed on MI355X (cold weights,
+// the launches included, us; before: the register-streaming GEMV up to 16 rows, hipBLASLt and separate
+// SiLU / add + norm kernels above):
+//   rows               1             4            16            32            48            64
+//   QKV           11.2 / 10.3   12.0 / 10.4   14.7 / 10.7   11.4 / 10.9   15.4 / 12.1   15.3 / 13.0
+//   O + norm      12.6 / 11.5   15.3 / 11.7   24.2 / 12.5   15.7 / 13.1   15.8 / 14.6   17.8 / 14.9
+//   gate/up       30.4 / 22.8   31.8 / 22.3   37.5 / 22.3   29.1 / 23.3   32.6 / 25.8   30.4 / 28.3
+//   down + norm   18.8 / 16.9   22.4 / 17.4   33.8 / 18.7   23.4 / 21.1   23.7 / 21.8   31.4 / 23.3
+//   lm_head        181 / 122     196 / 122     232 / 128     172 / 144     159 / 160     181 / 175
+// About 5 us of each are the launch and the first loads' latency; the lm_head streams at 6.4 TB/s. Equal
 // shares of K x tiles for every workgroup (stream-K over 64-row tiles) cost the partials' round trips:
 // 13.5 us for QKV at M = 1, 14.8 at 32. The norm by the last workgroup of the same launch took 3 us more
-// than its own launch (two hand-offs). Above 64 rows x's share of the loads grows past what hipBLASLt's
-// larger tiles need (80 rows: O 18.6 against 16.1).
+// than its own launch (two hand-offs).
+// Above 64 rows x's share of the loads grows (every workgroup reads all of it) and hipBLASLt's larger
+// tiles win where nothing else is saved (QKV 15.0 / 15.5 at 80 rows, 18.5 / 20.4 at 131). With the
+// epilogues a launch and a pass over the product go too (hipBLASLt and the separate kernel / this one):
+//   rows              65            80            96           112           128           144
+//   gate/up      37.3 / 35.0   37.3 / 36.1   36.1 / 34.5   35.9 / 37.5   34.2 / 38.4   44.3 / 41.1
+//   O + norm     18.8 / 16.5   19.1 / 16.9   19.6 / 18.5   19.1 / 18.9   19.5 / 19.5   18.0 / 20.9
+//   down + norm  31.0 / 26.2   32.1 / 27.5   34.4 / 26.9   35.6 / 28.3   36.0 / 28.7   32.6 / 31.4
+// so the sums are taken up to 128 rows and SiLU up to 96 (from 129 to 160 rows it is 2 - 7% ahead again,
+// hipBLASLt's time being a staircase of its tile heights: not worth a second range). A different first stage for each workgroup, so that they do not
+// read the same lines of x at once, gained nothing up to 64 rows and cost 0.5 us in O and down above.
 //
 // MFMA 16x16x32: A = 16 weight rows, B = 16 activation rows (x^T), both read from LDS. The 8 waves
 // split a stage into (k-steps of 32) x (weight tiles), and every wave multiplies its weight fragments
@@ -291,13 +307,14 @@ struct Plan {
 
 // The tiling of one product. N: rows of W (mode SILU: 2 I). Returns false for shapes not taken.
 bool plan_for(int mode, int M, int N, int K, Plan& p) {
-  if (M < 1 || M > 64 || N < 1 || K < 64 || K % 64 != 0) return false;
+  if (M < 1 || M > (mode == lin::OUT ? 64 : mode == lin::SILU ? 96 : 128) || N < 1 || K < 64 || K % 64 != 0) return false;
   if ((long long)N * K >= (1ll << 30) || (long long)M * K >= (1ll << 30)) return false;   // buffer offsets
   if (mode == lin::SILU && N % 2 != 0) return false;
   const int G = cu_count();
   if (G <= 0) return false;
   p.nout = mode == lin::SILU ? N / 2 : N;
   p.bmt = (M + 15) / 16;
+  if (p.bmt > 4) p.bmt += p.bmt & 1;                                   // 6, 8: rows past M cost no loads
   const int per16 = mode == lin::SILU ? 8 : 16;                        // outputs of a 16-row weight tile
   // S: parts of K (PART: the sums meet in the norm's launch); nv: outputs of S workgroups, in tiles of at
   // most 128 rows
@@ -365,8 +382,12 @@ int launch(const Plan& p, const void* x, const void* W, void* y, int M, int N, i
     case 1: return launch_nt<1, MODE>(a, p, stream);
     case 2: return launch_nt<2, MODE>(a, p, stream);
     case 3: return launch_nt<3, MODE>(a, p, stream);
-    default: return launch_nt<4, MODE>(a, p, stream);
+    case 4: return launch_nt<4, MODE>(a, p, stream);
   }
+  if constexpr (MODE != lin::OUT)
+    if (p.bmt == 6) return launch_nt<6, MODE>(a, p, stream);
+  if constexpr (MODE == lin::PART) return launch_nt<8, MODE>(a, p, stream);
+  return (int)hipErrorInvalidValue;
 }
 
 }  // namespace

@@ -26,6 +26,10 @@ from ._lib import check, lib
 
 BM_MAX = 16  # largest activation-row count the skinny GEMV takes (fused.py:838 BM_MAX role)
 LIN_MAX = 64  # largest activation-row count of the weight-streaming linear kernels
+# With SiLU * up, and with the residual add + norm, they stay the faster ones further, since those passes
+# go with the product (measured, the table in csrc/linear.hip).
+LIN_SILU_MAX = 96
+LIN_NORM_MAX = 128
 NORM_MAX = 4096  # longest row the row-norm kernels take
 # Smallest row count sent to the library's own hipBLASLt call: everything past the skinny kernels.
 # (F.linear asks hipBLASLt's heuristic again on every call, 21 us of host time against 6.)
@@ -142,15 +146,16 @@ class HipOps:
         return (self.use_gemv and 1 <= M <= BM_MAX and _bf16_ok(x, w) and K % 8 == 0
                 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
-    def _linear_ok(self, x, w):
+    def _linear_ok(self, x, w, rows=LIN_MAX):
         """Whether the weight-streaming linear kernels take x @ w^T: the kernels of choice up to
-        LIN_MAX rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt. Operands that need a
+        `rows` rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt. Operands that need a
         gradient keep F.linear above the GEMV's rows."""
         M, K = x.shape
-        return (self.use_gemv and 1 <= M <= LIN_MAX and w.dim() == 2 and w.shape[1] == K
+        return (self.use_gemv and 1 <= M <= rows and w.dim() == 2 and w.shape[1] == K
                 and (M <= BM_MAX or not _wants_grad(x, w))
                 and _bf16_ok(x, w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-                and bool(self.L.dd_linear_supported(M, w.shape[0], K)))
+                and x.numel() < 1 << 30
+                and bool(self.L.dd_linear_supported(min(M, LIN_MAX), w.shape[0], K)))
 
     def _gemm_ok(self, x, w):
         """Prefill-sized bf16 products go to the library's hipBLASLt GEMM (dd_gemm_bf16) with the
@@ -251,7 +256,7 @@ class HipOps:
         return out
 
     def gate_up_silu(self, x, wgu):
-        if wgu.shape[0] % 2 == 0 and self._linear_ok(x, wgu):
+        if wgu.shape[0] % 2 == 0 and self._linear_ok(x, wgu, LIN_SILU_MAX):
             M, K = x.shape
             I = wgu.shape[0] // 2
             out = torch.empty((M, I), dtype=x.dtype, device=x.device)
@@ -270,7 +275,8 @@ class HipOps:
     def linear_add_norm(self, x, w, h, lnw):
         """hn = h + x @ w^T ; returns (hn, rmsnorm(hn, lnw))"""
         if (w.shape[0] <= NORM_MAX and h.shape == (x.shape[0], w.shape[0])
-                and lnw.numel() == w.shape[0] and _bf16_ok(h, lnw) and self._linear_ok(x, w)):
+                and lnw.numel() == w.shape[0] and _bf16_ok(h, lnw)
+                and self._linear_ok(x, w, LIN_NORM_MAX)):
             M, K = x.shape
             N = w.shape[0]
             ws = torch.empty(self.L.dd_linear_add_rmsnorm_ws_bytes(M, N, K) // 4,

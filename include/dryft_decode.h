@@ -83,10 +83,12 @@ size_t dd_gemv_add_rmsnorm_ws_bytes(int M, int N, int K, int splitk);
 int dd_gate_up_silu(const void* x, const void* Wgu, void* out, int M, int I, int K,
                     hipStream_t stream);
 
-/* Skinny linear layers, 1 <= M <= 64 rows (K % 64 == 0, N * K < 2^30; x, W, ws and the products
- * 16-byte aligned): the products and epilogues of dd_gemv / dd_gate_up_silu / dd_gemv_add_rmsnorm
- * with the weights streamed through LDS, every workgroup an equal share of the outputs.
- * dd_linear_supported: 1 when the shape is taken (N: rows of W, so 2 I for dd_linear_silu).
+/* Skinny linear layers, 1 <= M <= 64 rows (dd_linear_silu 96, dd_linear_add_rmsnorm 128; K % 64 == 0,
+ * N * K < 2^30; x, W, ws and the products 16-byte aligned): the products and epilogues of dd_gemv /
+ * dd_gate_up_silu / dd_gemv_add_rmsnorm with the weights streamed through LDS, every workgroup an equal
+ * share of the outputs.
+ * dd_linear_supported: 1 when dd_linear takes the shape (N: rows of W, so 2 I for dd_linear_silu); the
+ * other two take the same N and K up to their own row limits while M * K < 2^30.
  * dd_linear_add_rmsnorm is two launches (N <= 4096): the product as fp32 sums in ws
  * (dd_linear_add_rmsnorm_ws_bytes bytes), then the residual add and the norm. No counters: calls on
  * different streams need only workspaces of their own.

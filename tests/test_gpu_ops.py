@@ -286,6 +286,31 @@ def test_streamed_linear_exact(small, M, N, K):
         assert ((y.float().cpu() - norm).abs() <= 2 ** -8 * norm.abs() + 1e-30).all()
 
 
+# above 64 rows: the edges of the 32-row steps and of the ranges of SiLU (96) and the sums (128), a ragged last tile
+@pytest.mark.parametrize("M", [65, 80, 96, 97, 128, 129])
+@pytest.mark.parametrize("N,K", [(72, 256), (1000, 192), (2560, 1024), (20002, 64), (40000, 128)])
+def test_streamed_epilogues_exact(small, M, N, K):
+    """The products of test_streamed_linear_exact (whole numbers below 256) through the epilogues."""
+    hip = small[1]
+    g = torch.Generator().manual_seed(M * 7 + N)
+    x = torch.randint(-1, 2, (M, K), generator=g).to(BF)
+    w = torch.randint(-1, 2, (N, K), generator=g).to(BF)
+    ref = x.float() @ w.float().t()
+    assert ref.abs().max() < 256
+    gu, up = ref.chunk(2, -1)
+    want = (torch.nn.functional.silu(gu).to(BF).float() * up).to(BF).float()
+    got = hip.gate_up_silu(x.cuda(), w.cuda()).cpu().float()
+    assert ((got - want).abs() <= 2 ** -6 * want.abs() + 1e-30).all()     # two bf16 roundings, as above
+    if N <= 4096:
+        h = torch.randint(-64, 65, (M, N), generator=g).to(BF)
+        lnw = torch.ones(N, dtype=BF)
+        hn, y = hip.linear_add_norm(x.cuda(), w.cuda(), h.cuda(), lnw.cuda())
+        want = (h.float() + ref).to(BF).float()
+        assert torch.equal(hn.float().cpu(), want)
+        norm = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + hip.e.eps)
+        assert ((y.float().cpu() - norm).abs() <= 2 ** -8 * norm.abs() + 1e-30).all()
+
+
 def test_linear_dtype_and_layout_fallback(small):
     """test_linear_precision.py:16-27: fp32/fp16/non-contiguous inputs route to F.linear."""
     _, hip, _ = small
