@@ -530,18 +530,21 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[t][i]);
     mx = max_rows32(mx);                                        // raw scores
-    const bool up = mx > m_run;                                 // the first block: key 0 is always seen
+    const bool up = mx > m_run;
+    // A row's maximum is -inf until it meets a finite score (key 0 is always seen, but its score may
+    // overflow): 0 in its place gives such keys weight 0 and no inf - inf.
+    auto finite = [](float m) { return m == -INFINITY ? 0.f : m; };
     if (__any(up)) {
-      const float m_new = up ? mx : m_run;
-      const float alpha = exp2_hw((m_run - m_new) * scale_log2);   // 1 in rows that keep theirs
+      const float m_old = m_run;
+      m_run = up ? mx : m_run;
+      const float alpha = exp2_hw((m_old - finite(m_run)) * scale_log2);   // 1 in rows that keep theirs
       l_run *= alpha;
 #pragma unroll
       for (int d = 0; d < 4; ++d)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[d][i] *= alpha;
-      m_run = m_new;
     }
-    const float mscl = m_run * scale_log2;
+    const float mscl = finite(m_run) * scale_log2;
     float ps[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 2; ++t)

@@ -197,6 +197,35 @@ def test_attn_prefill_dma_equals_register_staging(cuda):
         assert torch.equal(ol, dma[last.cuda()])
 
 
+@pytest.mark.parametrize("lens,NH", [((130, 65, 200), 32), ((4165,), 4)])
+def test_attn_prefill_first_keys_overflow(cuda, lens, NH):
+    """Finite q and k whose products overflow to -inf in a row's first 64 keys (every odd token's, so that
+    a wave holds rows of both kinds): those keys have weight 0 and the later ones count as ever. The 4-wave
+    and (one prompt of 4,096 tokens or more) the 8-wave kernel."""
+    NKV, B, cap = NH // 4, len(lens), max(lens) + 3
+    hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
+    starts = _starts(lens)
+    T = starts[-1]
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(T, NH, HD, generator=g).to(BF)
+    kc = torch.randn(B, NKV, cap, HD, generator=g).to(BF)
+    vc = torch.randn(B, NKV, cap, HD, generator=g).to(BF)
+    q[:, :, 0], kc[:, :, :, 0] = 0, 0
+    for b in range(B):
+        q[starts[b] + 1:starts[b + 1]:2, :, 0] = 1e25
+    kc[:, :, :64, 0] = -1e25
+    ss = torch.tensor(starts, dtype=torch.int32).cuda()
+    out = hip.attn_prefill_packed(q.cuda(), kc.cuda(), vc.cuda(), ss, B, T).view(T, NH, HD).double().cpu()
+    for b, n in enumerate(lens):
+        # odd tokens below 64 see overflowed scores only: no value to compare
+        rows = torch.tensor([p for p in (*range(min(n, 300)), *range(300, n, 61), n - 1) if p % 2 == 0 or p > 64])
+        for h in range(0, NH, max(1, NH // 4)):
+            s = q[starts[b] + rows, h].double() @ kc[b, h // 4, :n].double().T * HD ** -0.5
+            s = s.masked_fill(torch.arange(n)[None] > rows[:, None], float("-inf"))
+            d = (out[starts[b] + rows, h] - torch.softmax(s, -1) @ vc[b, h // 4, :n].double()).abs().max().item()
+            assert d < 0.02, (b, h, d)
+
+
 def test_attn_prefill_more_prompts_than_a_grid_dimension(cuda):
     """65,600 prompts of one token (a grid's second dimension ends at 65,535): each row is its own value."""
     hip = _hip(fake_engine(nh=4, nkv=1, hd=HD, rope_len=16))
