@@ -13,7 +13,7 @@ import torch  # noqa: F401  (load order: see module docstring)
 
 LIB_NAME = "libdryft_decode.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -23,6 +23,7 @@ _Z = ctypes.c_size_t
 # name -> (restype, argtypes)
 _SIGS = {
     "dd_abi_version": (_I, []),
+    "dd_capture_id": (_I, [_P, ctypes.POINTER(ctypes.c_ulonglong)]),
     "dd_rmsnorm": (_I, [_P, _P, _P, _I, _I, _F, _P]),
     "dd_add_rmsnorm": (_I, [_P, _P, _P, _P, _P, _I, _I, _F, _P]),
     "dd_gemv": (_I, [_P, _P, _P, _I, _I, _I, _I, _P, _P, _P]),

@@ -9,7 +9,7 @@
 
 namespace dd {
 
-constexpr int DD_ABI_VERSION = 16;
+constexpr int DD_ABI_VERSION = 17;
 
 inline bool aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
 

@@ -349,6 +349,16 @@ using namespace dd;
 
 DD_API int dd_abi_version(void) { return DD_ABI_VERSION; }
 
+DD_API int dd_capture_id(hipStream_t stream, unsigned long long* id) {
+  DD_REQUIRE(id);
+  *id = 0;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  unsigned long long cap = 0;
+  const hipError_t e = hipStreamGetCaptureInfo(stream, &st, &cap);
+  if (e == hipSuccess && st == hipStreamCaptureStatusActive) *id = cap;
+  return (int)e;
+}
+
 DD_API int dd_gemv_splitk(int M, int N, int K) { return pick_splitk(M, N, K); }
 
 // Bytes of fp32 partials for a split (at least one split's worth, which the fused

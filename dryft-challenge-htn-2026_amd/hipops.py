@@ -15,6 +15,7 @@ allocated with ``torch.empty`` (so they come from the graph pool under capture).
 status raises ``RuntimeError``.
 """
 import bisect
+import ctypes
 import functools
 import json
 import os
@@ -35,6 +36,9 @@ NORM_MAX = 4096  # longest row the row-norm kernels take
 # (F.linear asks hipBLASLt's heuristic again on every call, 21 us of host time against 6.)
 GEMM_MIN_M = LIN_MAX + 1
 GEMM_WS_MAX = 8  # hipBLASLt workspaces an ops object keeps (64 MiB each)
+COUNTERS = 4096  # counters of an array (more where a call needs more)
+COUNTERS_MAX = 64  # counter arrays that an ops object keeps for its streams
+GRAPHS = 16  # and for graph captures
 
 
 def _ptr(t):
@@ -126,20 +130,44 @@ class HipOps:
         self.use_gemv = use_gemv
         assert e.hd & (e.hd - 1) == 0 and e.hd >= 2
         self.L = lib()  # raises when the library is missing: no silent fallback
-        self._counters = None
+        self._counters = {}  # zeroed counters by (device, stream), at most COUNTERS_MAX
+        self._graph_counters = 0, {}  # the same of the graph capture with this id
         self._gemm_ws = {}  # hipBLASLt workspaces by (device, stream), at most GEMM_WS_MAX
         self._gemm_table = load_gemm_table()
         self._starts = {}
         self.err = torch.zeros(1, dtype=torch.int32, device=e.dev)
+        # counters for GRAPHS captures, each given out once. Like err and the tables they are there
+        # for work that is ordered after this (torch.cuda.graph waits for the device).
+        self._spares = torch.zeros((GRAPHS, COUNTERS), dtype=torch.int32, device=e.dev)
+        self._spare = list(self._spares)
 
     # ---------------------------------------------------------------- helpers
     def _zeroed_counters(self, n, dev):
-        """Zeroed int32 counters shared by every call on this stream (the kernels leave them
-        zero). Allocated once, outside graph capture, and grown only when a larger op needs it."""
-        c = self._counters
-        if c is None or c.numel() < n or c.device != dev:
-            self._counters = torch.zeros(max(n, 16384), dtype=torch.int32, device=dev)
-        return self._counters
+        """Zeroed int32 counters for a call on the current stream (the kernels leave them zero):
+        one array per stream, since calls that overlap must not share any, and graphs may run at
+        the same time, so each capture gets arrays of its own. Those are taken from the ones that
+        this object was made with (it has to outlive its graphs, as for ``err``); after them, or
+        for more counters, from the graph's pool, where the graph has to clear them first (1.4 us
+        a replay)."""
+        key = dev, _stream(dev)
+        if torch.cuda.is_current_stream_capturing():
+            capture = ctypes.c_ulonglong()
+            check(self.L.dd_capture_id(key[1], ctypes.byref(capture)), "dd_capture_id")
+            if self._graph_counters[0] != capture.value:
+                self._graph_counters = capture.value, {}
+            kept = self._graph_counters[1]
+            c = kept.get(key)
+            if c is None or c.numel() < n:
+                fits = n <= COUNTERS and dev == self.err.device
+                c = kept[key] = (self._spare.pop() if fits and self._spare else
+                                 torch.zeros(max(n, COUNTERS), dtype=torch.int32, device=dev))
+            return c
+        c = self._counters.get(key)
+        if c is None or c.numel() < n:
+            if c is None and len(self._counters) >= COUNTERS_MAX:
+                self._counters.clear()  # each goes back to the allocator, in its stream's order
+            c = self._counters[key] = torch.zeros(max(n, COUNTERS), dtype=torch.int32, device=dev)
+        return c
 
     def _gemv_ok(self, x, w):
         M, K = x.shape

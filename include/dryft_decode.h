@@ -42,6 +42,10 @@ extern "C" {
 /* ABI version (bumped on any signature change). */
 int dd_abi_version(void);
 
+/* *id: the graph capture that `stream` is in (its unique id), 0 outside one. Launches nothing. For
+ * hosts that keep counters or workspaces per stream: a captured call's belong to its graph. */
+int dd_capture_id(hipStream_t stream, unsigned long long* id);
+
 /* y[m] = rmsnorm(x[m]) * w, m < M, row length N (N <= 4096).
  * Replaces TritonOps.rms (fused.py:894-895; kernel fused.py:152-172), reference
  * _TorchOps.rms / _rms (engine.py:107-110, 134-135). */

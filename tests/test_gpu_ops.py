@@ -481,6 +481,47 @@ def test_attn_equal_shares(cuda, NH, NKV, W, cap, lens):
     assert d < 0.02, d
 
 
+@torch.inference_mode()
+def test_attn_streams_and_graphs_at_once(cuda):
+    """Short contexts that lie in several workgroups (65 keys in a 256-slot cache), eagerly on two streams
+    and in two replayed graphs at the same time: every result has the bits of a call by itself."""
+    NH, NKV, HD, cap, B = 32, 8, 128, 256, 3
+    hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
+    g = torch.Generator().manual_seed(9)
+    pos = torch.tensor([64, 127, 70]).cuda()
+    sets = [[torch.randn(*s, generator=g).to(BF).cuda() for s in
+             ((B, NKV, 1, NH // NKV, HD), (B, NKV, cap, HD), (B, NKV, cap, HD))] for _ in range(2)]
+    alone = [hip.attn_decode(*t, pos) for t in sets]
+    streams = [torch.cuda.Stream() for _ in sets]
+    torch.cuda.synchronize()
+    outs = [[], []]
+    for _ in range(50):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                outs[i].append(hip.attn_decode(*sets[i], pos))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(o, alone[i]) for o in outs[i])
+    graphs = []
+    for i, t in enumerate(sets):
+        if i == 1:
+            hip._spare.clear()                              # a graph that clears its own
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            graphs.append((graph, [hip.attn_decode(*t, pos) for _ in range(4)]))
+    for _ in range(3):
+        for _, out in graphs:
+            for o in out:
+                o.zero_()
+        torch.cuda.synchronize()
+        for s, (graph, _) in zip(streams, graphs):
+            with torch.cuda.stream(s):
+                graph.replay()
+        torch.cuda.synchronize()
+        for i, (_, out) in enumerate(graphs):
+            assert all(torch.equal(o, alone[i]) for o in out)
+
+
 # ------------------------------------------------------------------------ argmax
 def test_argmax_rules_and_pos(cuda):
     from dryft_amd.hipops import HipOps

@@ -86,3 +86,41 @@ def test_qkv_head_grouped_order(nh, nkv):
     grouped = torch.tensor(order).view(1, 1, n)
     assert sorted(order) == list(range(n))
     assert torch.equal(FusedStep.qkv_natural(grouped, nh, nkv).view(-1), torch.arange(n))
+
+
+def test_op_counters_are_not_shared(monkeypatch):
+    """Calls on two streams, and calls of two graph captures, never get the same counters (calls that
+    overlap would race on them); one stream, and one capture on one stream, keeps its own."""
+    from dryft_amd import hipops
+    at = {"stream": 1, "capture": 0}
+
+    class Lib:
+        @staticmethod
+        def dd_capture_id(stream, out):
+            out._obj.value = at["capture"]
+            return 0
+
+    ops = object.__new__(hipops.HipOps)
+    ops.L, ops._counters, ops._graph_counters = Lib, {}, (0, {})
+    ops.err = torch.zeros(1)
+    ops._spares = torch.zeros(3, hipops.COUNTERS, dtype=torch.int32)
+    ops._spare = list(ops._spares)
+    monkeypatch.setattr(hipops, "_stream", lambda dev: at["stream"])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: at["capture"] != 0)
+
+    def get(stream, capture, n=8):
+        at.update(stream=stream, capture=capture)
+        c = ops._zeroed_counters(n, torch.device("cpu"))
+        assert c.numel() >= n and not c.any()
+        return c
+
+    a, b = get(1, 0), get(2, 0)
+    g1, g1_side, = get(3, 7), get(4, 7)
+    assert get(3, 7) is g1                          # before another capture begins
+    g2 = get(3, 8)
+    assert get(1, 0) is a and get(2, 0) is b and get(3, 8) is g2
+    kept = [a, b, g1, g1_side, g2, get(3, 0), get(1, 0, 20000), get(3, 9), get(3, 9, 20000), get(3, 10)]
+    assert len({c.data_ptr() for c in kept}) == len(kept)
+    for s in range(300):                            # bounded
+        get(100 + s, 0)
+    assert len(ops._counters) <= hipops.COUNTERS_MAX
