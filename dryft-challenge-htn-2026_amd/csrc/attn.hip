@@ -386,9 +386,9 @@ attn_stream_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc, cons
       for (int k = 0; k < 4; ++k)                 // keys past the last read 0 (masked)
         kr[t][k] = __builtin_amdgcn_raw_buffer_load_b128(krs, k0 + t * 16 * HD * 2 + k * 64, 0, 2);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {                 // 4 keys each; past the last: a copy of the last (weight 0)
-      const int key = min(j * 32 + i * 4 + vr, L - 1);
-      const unsigned off = (unsigned)key * HD * 2 + ((l16 ^ (2 * ((i * 4 + vr) & 7))) * 16);
+    for (int i = 0; i < 8; ++i) {                 // 4 keys each; keys past the last: zeros (out of the range)
+      const unsigned key = j * 32 + i * 4 + vr;
+      const unsigned off = key * HD * 2 + ((l16 ^ (2 * ((i * 4 + vr) & 7))) * 16);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           vrs, (__attribute__((address_space(3))) void*)(size_t)(lds_v + buf * (32 * HD * 2) + i * 1024), 16, off, 0, 0, 2);
     }

@@ -481,6 +481,28 @@ def test_attn_equal_shares(cuda, NH, NKV, W, cap, lens):
     assert d < 0.02, d
 
 
+@pytest.mark.parametrize("lens", [[33, 64, 577, 1, 640], [8190]])
+def test_attn_infinite_newest_value(cuda, lens):
+    """An infinite value of the newest key makes that dim infinite, and nothing NaN: slots past it count
+    as zeros, which they are."""
+    NH, NKV, HD, cap, B = 32, 8, 128, max(lens) + 2, len(lens)
+    hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
+    g = torch.Generator().manual_seed(B)
+    kc, vc = (torch.randn(B, NKV, cap, HD, generator=g).to(BF) for _ in range(2))
+    q = torch.randn(B, NKV, 1, NH // NKV, HD, generator=g).to(BF)
+    for b, n in enumerate(lens):
+        kc[b, :, n:] = vc[b, :, n:] = 0
+        vc[b, :, n - 1, 5] = 0
+    pos = torch.tensor(lens) - 1
+    ref = attn_reference_fp64(q, kc, vc, pos, 1, NH, NKV, HD).view(B, NH, HD)
+    for b, n in enumerate(lens):
+        vc[b, :, n - 1, 5] = float("inf")
+    out = hip.attn_decode(q.cuda(), kc.cuda(), vc.cuda(), pos.cuda()).double().cpu().view(B, NH, HD)
+    assert (out[:, :, 5] == float("inf")).all()
+    out[:, :, 5] = ref[:, :, 5]
+    assert (out - ref).abs().max().item() < 0.02
+
+
 @torch.inference_mode()
 def test_attn_streams_and_graphs_at_once(cuda):
     """Short contexts that lie in several workgroups (65 keys in a 256-slot cache), eagerly on two streams
