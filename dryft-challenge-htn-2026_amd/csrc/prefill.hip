@@ -421,7 +421,7 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
   const unsigned lds_k = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) bf16*)shk);
   const unsigned lds_v = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) bf16*)shv);
   // DMA: instruction i fills rows 4 i .. 4 i + 3 of a buffer; wave w issues IPW of them. Rows past the
-  // prompt repeat its last key (masked); blocks past the last repeat it (not used).
+  // prompt are out of the range and land as zeros (masked, 0 x 0); blocks past the last repeat it (not used).
   auto dma = [&](rsrc_t r, unsigned voff, unsigned lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "s"(lds) : "m0", "memory");
   };
@@ -431,7 +431,7 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
 #pragma unroll
     for (int i = 0; i < IPW; ++i) {
       const int r = drow + 4 * i;
-      dma(kr, (unsigned)min(key0 + r, len - 1) * HD * 2 + (dc ^ (r & 15)) * 16, lds_k + buf * (BUF * 2) + (IPW * wave + i) * 1024);
+      dma(kr, (unsigned)(key0 + r) * HD * 2 + (dc ^ (r & 15)) * 16, lds_k + buf * (BUF * 2) + (IPW * wave + i) * 1024);
     }
   };
   auto issue_v = [&](int j, int buf) {
@@ -439,7 +439,7 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
 #pragma unroll
     for (int i = 0; i < IPW; ++i) {
       const int r = drow + 4 * i;
-      dma(vr, (unsigned)min(key0 + r, len - 1) * HD * 2 + (dc ^ (4 * (r & 3))) * 16, lds_v + buf * (BUF * 2) + (IPW * wave + i) * 1024);
+      dma(vr, (unsigned)(key0 + r) * HD * 2 + (dc ^ (4 * (r & 3))) * 16, lds_v + buf * (BUF * 2) + (IPW * wave + i) * 1024);
     }
   };
   auto phase_end = [&] {

@@ -226,6 +226,30 @@ def test_attn_prefill_first_keys_overflow(cuda, lens, NH):
             assert d < 0.02, (b, h, d)
 
 
+@pytest.mark.parametrize("lens,NH", [((33, 100, 64, 1), 32), ((4165,), 4)])
+def test_attn_prefill_infinite_last_value(cuda, lens, NH):
+    """An infinite value of a prompt's last key makes that dim of the last query infinite, and nothing
+    NaN, in a full pass and with last_only."""
+    NKV, B, cap = NH // 4, len(lens), max(lens) + 3
+    hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
+    starts = _starts(lens)
+    T = starts[-1]
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(T, NH, HD, generator=g).to(BF).cuda()
+    kc, vc = (torch.randn(B, NKV, cap, HD, generator=g).to(BF).cuda() for _ in range(2))
+    ss = torch.tensor(starts, dtype=torch.int32).cuda()
+    last = torch.tensor(starts[1:]).cuda() - 1
+    plain = hip.attn_prefill_packed(q, kc, vc, ss, B, T)[last].view(B, NH, HD)
+    for b, n in enumerate(lens):
+        vc[b, :, n - 1, 5] = float("inf")
+    for out in (hip.attn_prefill_packed(q, kc, vc, ss, B, T)[last],
+                hip.attn_prefill_packed(q[last].contiguous(), kc, vc, ss, B, T, last_only=True)):
+        out = out.view(B, NH, HD)
+        assert (out[:, :, 5] == float("inf")).all()
+        for d in (slice(0, 5), slice(6, None)):
+            assert torch.equal(out[:, :, d], plain[:, :, d])
+
+
 def test_attn_prefill_more_prompts_than_a_grid_dimension(cuda):
     """65,600 prompts of one token (a grid's second dimension ends at 65,535): each row is its own value."""
     hip = _hip(fake_engine(nh=4, nkv=1, hd=HD, rope_len=16))
