@@ -482,12 +482,13 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
   };
   // O^T += V^T.P^T of a block, and (QK) S^T of the next one. The operand reads run two key steps ahead of
   // their MFMAs: left alone, the compiler reads each operand right before its MFMA and waits for it.
-  auto pv = [&](int bv, int bk, auto with_qk) {
+  auto pv = [&](int bv, int bk, auto with_qk, auto nsteps) {
     constexpr bool QK = decltype(with_qk)::value;
+    constexpr int NS = decltype(nsteps)::value;                 // 16-key steps
     const bf16* vb = shv + bv * BUF;
-    u32x4 vf[4][4];
+    u32x4 vf[NS][4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < NS; ++t)
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
         const u32x2 lo = lds_read_tr16(&vb[t * 16 * HD + va[d]]);
@@ -495,13 +496,13 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
         vf[t][d] = u32x4{lo.x, lo.y, hi.x, hi.y};
       }
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < NS; ++t)
 #pragma unroll
       for (int d = 0; d < 4; ++d) acc[d] = mfma32(vf[t][d], pk[t], acc[d]);
     if constexpr (QK) qk(bk);
     __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);         // V of steps 0 and 1
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < (NS - 2) * 4; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);        // V of steps 2 and 3
     }
@@ -559,7 +560,14 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
   };
 
   const std::integral_constant<bool, true> next{};
-  const std::integral_constant<bool, false> final{};
+  const std::integral_constant<int, 4> all{};
+  // The last block: a wave whose queries lie in its first half leaves the second, whose keys they do not
+  // see, out, so that no infinite value there meets their weight 0.
+  auto pv_last = [&](int bv) {
+    const std::integral_constant<bool, false> final{};
+    if ((p0 & 32) || late) pv(bv, 0, final, all);
+    else pv(bv, 0, final, std::integral_constant<int, 2>{});
+  };
   issue_k(0, 0);
   issue_k(1, 1);
   issue_v(0, 0);
@@ -573,12 +581,12 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
       phase_end();                                              // block j - 1 is read, V(j) and K(j + 1) landed
       issue_k(j + 2, j & 1);
       issue_v(j + 1, (j + 1) & 1);
-      pv(j & 1, (j + 1) & 1, next);
+      pv(j & 1, (j + 1) & 1, next, all);
     }
     softmax(nblk - 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     phase_end();
-    pv((nblk - 1) & 1, 0, final);
+    pv_last((nblk - 1) & 1);
   } else {
     issue_k(2, 2);
     issue_v(1, 1);
@@ -598,14 +606,14 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
         phase_end();
         issue_k(j + 3, b0);
         issue_v(j + 2, b2);
-        pv(b0, b1, next);
+        pv(b0, b1, next, all);
         phase_end();
         turn();
       }
       softmax(nblk - 1);
       landed();
       phase_end();
-      pv(b0, b1, final);
+      pv_last(b0);
       phase_end();
     } else {
       phase_end();
@@ -617,14 +625,14 @@ flash_prefill_pp_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc,
         issue_v(j + 2, b2);
         softmax(j);
         phase_end();
-        pv(b0, b1, next);
+        pv(b0, b1, next, all);
         landed();
         phase_end();
         turn();
       }
       softmax(nblk - 1);
       phase_end();
-      pv(b0, b1, final);
+      pv_last(b0);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // no load into LDS outlives the wave

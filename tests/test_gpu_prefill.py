@@ -250,6 +250,24 @@ def test_attn_prefill_infinite_last_value(cuda, lens, NH):
             assert torch.equal(out[:, :, d], plain[:, :, d])
 
 
+@pytest.mark.parametrize("n,NH,key", [(130, 32, 40), (130, 32, 100), (4165, 4, 40), (4165, 4, 4136)])
+def test_attn_prefill_infinite_value_stays_in_its_half_block(cuda, n, NH, key):
+    """An infinite value reaches no query of an earlier 32-key step: their bits stay (its own step's
+    earlier queries meet it with weight 0, which is NaN)."""
+    NKV = NH // 4
+    hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
+    g = torch.Generator().manual_seed(key)
+    q = torch.randn(n, NH, HD, generator=g).to(BF).cuda()
+    kc, vc = (torch.randn(1, NKV, n, HD, generator=g).to(BF).cuda() for _ in range(2))
+    ss = torch.tensor([0, n], dtype=torch.int32).cuda()
+    plain = hip.attn_prefill_packed(q, kc, vc, ss, 1, n)
+    vc[:, :, key, 5] = float("inf")
+    out = hip.attn_prefill_packed(q, kc, vc, ss, 1, n)
+    rows = key // 32 * 32
+    assert torch.equal(out[:rows], plain[:rows])
+    assert (out[key:].view(n - key, NH, HD)[:, :, 5] == float("inf")).all()
+
+
 def test_attn_prefill_more_prompts_than_a_grid_dimension(cuda):
     """65,600 prompts of one token (a grid's second dimension ends at 65,535): each row is its own value."""
     hip = _hip(fake_engine(nh=4, nkv=1, hd=HD, rope_len=16))
