@@ -88,7 +88,9 @@ def _wants_grad(*ts):
 
 
 def _bf16_ok(*ts):
-    return all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.is_cuda for t in ts)
+    dev = ts[0].get_device()
+    return all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.is_cuda
+               and t.get_device() == dev for t in ts)
 
 
 # -- torch helpers for the prefill branch (outside the decode step; same arithmetic as the
@@ -171,7 +173,8 @@ class HipOps:
 
     def _gemv_ok(self, x, w):
         M, K = x.shape
-        return (self.use_gemv and 1 <= M <= BM_MAX and _bf16_ok(x, w) and K % 8 == 0
+        return (self.use_gemv and 1 <= M <= BM_MAX and w.dim() == 2 and w.shape[1] == K
+                and _bf16_ok(x, w) and K % 8 == 0
                 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
     def _linear_ok(self, x, w, rows=LIN_MAX):
@@ -191,7 +194,7 @@ class HipOps:
         (it raises for mismatched shapes): other ranks, unaligned operands, operands that need a
         gradient. DD_TUNED_GEMM=0 keeps all of them there (diagnostics)."""
         return (x.dim() == w.dim() == 2 and x.shape[0] >= GEMM_MIN_M and x.shape[1] == w.shape[1]
-                and w.shape[0] > 0 and x.shape[1] > 0 and _bf16_ok(x, w) and x.device == w.device
+                and w.shape[0] > 0 and x.shape[1] > 0 and _bf16_ok(x, w)
                 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not _wants_grad(x, w)
                 and os.environ.get("DD_TUNED_GEMM", "1") != "0")
 
@@ -228,7 +231,7 @@ class HipOps:
     # ---------------------------------------------------------------- norms
     def rms(self, h, w):
         h = h.contiguous()
-        if not _bf16_ok(h, w):
+        if not _bf16_ok(h, w) or w.numel() != h.shape[-1]:
             return _rms_t(h, w, self.e.eps)
         M, N = h.reshape(-1, h.shape[-1]).shape
         y = torch.empty_like(h)
@@ -238,7 +241,8 @@ class HipOps:
 
     def add_rms(self, h, d, w):
         h, d = h.contiguous(), d.contiguous()
-        if not _bf16_ok(h, d, w):
+        if not (_bf16_ok(h, d, w) and h.numel() == d.numel()
+                and h.shape[-1] == d.shape[-1] == w.numel()):
             hn = h + d
             return hn, _rms_t(hn, w, self.e.eps)
         M, N = h.reshape(-1, h.shape[-1]).shape
@@ -252,7 +256,7 @@ class HipOps:
         gu = gu.contiguous()
         M, I2 = gu.shape
         out = torch.empty((M, I2 // 2), dtype=gu.dtype, device=gu.device)
-        if not _bf16_ok(gu):
+        if not _bf16_ok(gu) or I2 % 2:
             g, u = gu.chunk(2, -1)
             return F.silu(g) * u
         check(self.L.dd_silu_mul(_ptr(gu), _ptr(out), M, I2 // 2, _stream(gu.device)),
@@ -291,7 +295,7 @@ class HipOps:
             check(self.L.dd_linear_silu(_ptr(x), _ptr(wgu), _ptr(out), M, I, K, _stream(x.device)),
                   "dd_linear_silu")
             return out
-        if not self._gemv_ok(x, wgu):
+        if wgu.shape[0] % 2 or not self._gemv_ok(x, wgu):
             return self.silu_mul(self.linear(x, wgu))
         M, K = x.shape
         I = wgu.shape[0] // 2
@@ -303,7 +307,7 @@ class HipOps:
     def linear_add_norm(self, x, w, h, lnw):
         """hn = h + x @ w^T ; returns (hn, rmsnorm(hn, lnw))"""
         if (w.shape[0] <= NORM_MAX and h.shape == (x.shape[0], w.shape[0])
-                and lnw.numel() == w.shape[0] and _bf16_ok(h, lnw)
+                and lnw.numel() == w.shape[0] and _bf16_ok(x, h, lnw)
                 and self._linear_ok(x, w, LIN_NORM_MAX)):
             M, K = x.shape
             N = w.shape[0]
@@ -315,7 +319,8 @@ class HipOps:
                                                _ptr(y), M, N, K, self.e.eps, _ptr(ws),
                                                _stream(x.device)), "dd_linear_add_rmsnorm")
             return hn, y
-        if not (self._gemv_ok(x, w) and _bf16_ok(h, lnw)):
+        if not (self._gemv_ok(x, w) and _bf16_ok(x, h, lnw) and lnw.numel() == w.shape[0]
+                and h.shape[-1] == w.shape[0] and h.numel() == x.shape[0] * w.shape[0]):
             return self.add_rms(h, self.linear(x, w), lnw)
         M, K = x.shape
         N = w.shape[0]

@@ -235,8 +235,9 @@ def test_linear_keeps_what_only_f_linear_takes(small, M):
     x = torch.randint(-1, 2, (M, 192), generator=g).to(BF).cuda()
     w = torch.randint(-1, 2, (80, 192), generator=g).to(BF).cuda()
     ref = x.float() @ w.float().t()
-    with pytest.raises(RuntimeError):
-        hip.linear(x, w[:, :128].contiguous())
+    for rows in (1, 16, M):
+        with pytest.raises(RuntimeError):
+            hip.linear(x[:rows], w[:, :128].contiguous())
     wg = w.clone().requires_grad_()
     y = hip.linear(x, wg)
     assert torch.equal(y.float(), ref)

@@ -88,6 +88,65 @@ def test_qkv_head_grouped_order(nh, nkv):
     assert torch.equal(FusedStep.qkv_natural(grouped, nh, nkv).view(-1), torch.arange(n))
 
 
+class FakeLib:
+    """The library's side of HipOps on the CPU: sizes and choices as the library gives them, and the names
+    of the kernels that would have been launched."""
+
+    def __init__(self):
+        self.launched = []
+
+    def dd_linear_supported(self, M, N, K):
+        return int(1 <= M <= 64 and N >= 1 and K >= 64 and K % 64 == 0)
+
+    def __getattr__(self, name):
+        if name.endswith(("_bytes", "_splitk", "_counters")):
+            return lambda *a: 16
+        return lambda *a: self.launched.append(name) or 0
+
+
+@pytest.fixture
+def cpu_ops(monkeypatch):
+    """HipOps with its kernels replaced by a record of their launches, for CPU tensors."""
+    from types import SimpleNamespace
+    from dryft_amd import hipops
+    ops = object.__new__(hipops.HipOps)
+    ops.L, ops.e, ops.use_gemv, ops._gemm_table = FakeLib(), SimpleNamespace(eps=1e-6), True, {}
+    monkeypatch.setattr(hipops, "_bf16_ok", lambda *ts: all(
+        t.dtype == torch.bfloat16 and t.is_contiguous() for t in ts))
+    monkeypatch.setattr(hipops, "_stream", lambda dev: 0)
+    monkeypatch.setattr(ops, "_zeroed_counters", lambda n, dev: torch.zeros(n, dtype=torch.int32))
+    monkeypatch.setattr(ops, "_gemm_workspace", lambda dev, stream: torch.empty(16, dtype=torch.uint8))
+    return ops
+
+
+@pytest.mark.parametrize("K", [192, 200])
+@pytest.mark.parametrize("M", [1, 16, 17, 100])
+def test_mismatched_operands_reach_no_kernel(cpu_ops, M, K):
+    """Operands whose shapes do not fit raise, and nothing is launched that would read past them."""
+    b = lambda *s: torch.ones(s, dtype=torch.bfloat16)  # noqa: E731
+    x, w, h, n = b(M, K), b(80, K), b(M, 80), b(80)
+    ops = cpu_ops
+    products = [lambda: ops.linear(x, b(80, K - 64)), lambda: ops.linear(x, b(80, K + 8)),
+                lambda: ops.gate_up_silu(x, b(80, K - 64)), lambda: ops.linear_add_norm(x, b(80, K - 64), h, n)]
+    # here the product fits and may run; what follows it does not
+    epilogues = [lambda: ops.gate_up_silu(x, b(81, K)), lambda: ops.linear_add_norm(x, w, b(M, 72), n),
+                 lambda: ops.linear_add_norm(x, w, h, b(72)), lambda: ops.add_rms(h, b(M, 72), n),
+                 lambda: ops.add_rms(h, h, b(72)), lambda: ops.rms(h, b(72)), lambda: ops.silu_mul(b(M, 81))]
+    if M > 1:
+        epilogues.append(lambda: ops.linear_add_norm(x, w, b(M + 1, 80), n))
+    for calls, allowed in ((products, set()), (epilogues, {"dd_linear", "dd_gemv", "dd_gemm_bf16"})):
+        for call in calls:
+            ops.L.launched.clear()
+            with pytest.raises(RuntimeError):
+                call()
+            assert set(ops.L.launched) <= allowed, ops.L.launched
+    ops.L.launched.clear()
+    for call in (ops.linear, ops.gate_up_silu, lambda x, w: ops.linear_add_norm(x, w, h, n)):
+        call(x, w)
+        assert ops.L.launched or M > 16                   # what fits still runs
+        ops.L.launched.clear()
+
+
 def test_op_counters_are_not_shared(monkeypatch):
     """Calls on two streams, and calls of two graph captures, never get the same counters (calls that
     overlap would race on them); one stream, and one capture on one stream, keeps its own."""
