@@ -22,6 +22,9 @@ import os
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from ._lib import check, lib
 
@@ -82,15 +85,39 @@ def _stream(dev):
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
 
 
-def _wants_grad(*ts):
-    """Whether autograd would record an op on these: F.linear is differentiable, the kernels are not."""
-    return torch.is_grad_enabled() and any(t.requires_grad for t in ts)
+_TENSORS = frozenset((torch.Tensor, torch.nn.Parameter))
+_transform = torch._C._functorch.peek_interpreter_stack
+
+
+def _plain(x, w):
+    """Whether nothing but the caller takes part in an op on these. F.linear is seen by autograd, by
+    forward-mode and the other function transforms (vmap, jvp), by tracing and compiling, by
+    dispatch and function modes and by tensor subclasses; a kernel launch is seen by none."""
+    if torch.compiler.is_compiling() or type(x) not in _TENSORS or type(w) not in _TENSORS:
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return False
+    if (_transform() is not None or forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() or torch._C._is_tracing()):
+        return False
+    return (not torch._C._len_torch_function_stack()       # torch.set_default_device's is no watcher
+            or all(isinstance(m, DeviceContext) for m in _get_current_function_mode_stack()))
+
+
+def _recast(x):
+    """Whether F.linear would compute in another type under the current autocast: up to 255 rows the
+    products follow that (larger ones never have)."""
+    return (x.shape[0] < 256 and torch.is_autocast_enabled("cuda")
+            and torch.get_autocast_dtype("cuda") != x.dtype)
 
 
 def _bf16_ok(*ts):
     dev = ts[0].get_device()
-    return all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.is_cuda
-               and t.get_device() == dev for t in ts)
+    for t in ts:
+        if not (t.dtype == torch.bfloat16 and t.is_contiguous() and t.is_cuda
+                and t.get_device() == dev):
+            return False
+    return True
 
 
 # -- torch helpers for the prefill branch (outside the decode step; same arithmetic as the
@@ -179,11 +206,11 @@ class HipOps:
 
     def _linear_ok(self, x, w, rows=LIN_MAX):
         """Whether the weight-streaming linear kernels take x @ w^T: the kernels of choice up to
-        `rows` rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt. Operands that need a
-        gradient keep F.linear above the GEMV's rows."""
+        `rows` rows; other K go to the GEMV (M <= BM_MAX) or hipBLASLt. Above the GEMV's rows
+        F.linear keeps what is more than a computation (_plain, _recast)."""
         M, K = x.shape
         return (self.use_gemv and 1 <= M <= rows and w.dim() == 2 and w.shape[1] == K
-                and (M <= BM_MAX or not _wants_grad(x, w))
+                and (M <= BM_MAX or _plain(x, w) and not _recast(x))
                 and _bf16_ok(x, w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
                 and x.numel() < 1 << 30
                 and bool(self.L.dd_linear_supported(min(M, LIN_MAX), w.shape[0], K)))
@@ -191,11 +218,11 @@ class HipOps:
     def _gemm_ok(self, x, w):
         """Prefill-sized bf16 products go to the library's hipBLASLt GEMM (dd_gemm_bf16) with the
         solution the committed table names for the shape. F.linear keeps what the call cannot take
-        (it raises for mismatched shapes): other ranks, unaligned operands, operands that need a
-        gradient. DD_TUNED_GEMM=0 keeps all of them there (diagnostics)."""
+        (it raises for mismatched shapes): other ranks, unaligned operands, what is more than a
+        computation (_plain, _recast). DD_TUNED_GEMM=0 keeps all of them there (diagnostics)."""
         return (x.dim() == w.dim() == 2 and x.shape[0] >= GEMM_MIN_M and x.shape[1] == w.shape[1]
-                and w.shape[0] > 0 and x.shape[1] > 0 and _bf16_ok(x, w)
-                and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not _wants_grad(x, w)
+                and w.shape[0] > 0 and x.shape[1] > 0 and _plain(x, w) and _bf16_ok(x, w)
+                and not _recast(x) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
                 and os.environ.get("DD_TUNED_GEMM", "1") != "0")
 
     def _gemm_lib(self, x, w, solution=None):
@@ -205,7 +232,7 @@ class HipOps:
             solution = gemm_solution(self._gemm_table, N, K, M)
         stream = _stream(x.device)
         ws = self._gemm_workspace(x.device, stream)
-        y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        y = x.new_empty((M, N))
         check(self.L.dd_gemm_bf16(_ptr(x), _ptr(w), _ptr(y), M, N, K, _ptr(ws), ws.numel(),
                                   solution, stream), "dd_gemm_bf16")
         return y
@@ -226,14 +253,15 @@ class HipOps:
     def _gemm(self, x, w):
         """y = x . w^T on hipBLASLt with the table's solution for (N, K, M): a fixed choice per
         shape, so every process computes the same bits for the same operands."""
-        return self._gemm_lib(x.contiguous(), w.contiguous())
+        return self._gemm_lib(x, w)
 
     # ---------------------------------------------------------------- norms
     def rms(self, h, w):
         h = h.contiguous()
-        if not _bf16_ok(h, w) or w.numel() != h.shape[-1]:
+        N = h.shape[-1]
+        if not _bf16_ok(h, w) or w.numel() != N:
             return _rms_t(h, w, self.e.eps)
-        M, N = h.reshape(-1, h.shape[-1]).shape
+        M = h.numel() // max(N, 1)
         y = torch.empty_like(h)
         check(self.L.dd_rmsnorm(_ptr(h), _ptr(w), _ptr(y), M, N, self.e.eps, _stream(h.device)),
               "dd_rmsnorm")
@@ -241,11 +269,11 @@ class HipOps:
 
     def add_rms(self, h, d, w):
         h, d = h.contiguous(), d.contiguous()
-        if not (_bf16_ok(h, d, w) and h.numel() == d.numel()
-                and h.shape[-1] == d.shape[-1] == w.numel()):
+        N, n = h.shape[-1], h.numel()
+        if not (_bf16_ok(h, d, w) and n == d.numel() and N == d.shape[-1] == w.numel()):
             hn = h + d
             return hn, _rms_t(hn, w, self.e.eps)
-        M, N = h.reshape(-1, h.shape[-1]).shape
+        M = n // max(N, 1)
         hn = torch.empty_like(h)
         y = torch.empty_like(h)
         check(self.L.dd_add_rmsnorm(_ptr(h), _ptr(d), _ptr(w), _ptr(hn), _ptr(y), M, N,

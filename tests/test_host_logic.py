@@ -147,6 +147,66 @@ def test_mismatched_operands_reach_no_kernel(cpu_ops, M, K):
         ops.L.launched.clear()
 
 
+@pytest.mark.parametrize("M", [17, 64, 65, 255, 256, 300])
+def test_products_are_seen_by_what_watches_torch(cpu_ops, monkeypatch, M):
+    """Above 16 rows a product that gradients, function transforms, tracing, modes or tensor subclasses take
+    part in stays F.linear; a plain one, also under torch.set_default_device, is the kernels'."""
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    g = torch.Generator().manual_seed(M)
+    x, t = (torch.randint(-1, 2, (M, 64), generator=g).to(torch.bfloat16) for _ in range(2))
+    w = torch.randint(-1, 2, (48, 64), generator=g).to(torch.bfloat16)
+    linear, launched = cpu_ops.linear, cpu_ops.L.launched
+    y, dy = x @ w.t(), t @ w.t()
+
+    out, tangent = torch.func.jvp(lambda a: linear(a, w), (x,), (t,))
+    assert torch.equal(out, y) and torch.equal(tangent, dy)
+    with forward_ad.dual_level():
+        out = forward_ad.unpack_dual(linear(forward_ad.make_dual(x, t), w))
+        assert torch.equal(out.primal, y) and torch.equal(out.tangent, dy)
+    assert torch.equal(torch.vmap(lambda a: linear(a, w))(torch.stack([x, t])), torch.stack([y, dy]))
+    for mode in ("real", "fake"):
+        assert torch.equal(make_fx(lambda a, b: linear(a, b), tracing_mode=mode)(x, w)(t, w), dy)
+    assert torch.equal(torch.jit.trace(lambda a: linear(a, w), (x,), check_trace=False)(t), dy)
+    with FlopCounterMode(display=False) as flops:
+        linear(x, w)
+    assert flops.get_total_flops() == 2 * M * 48 * 64
+
+    seen = []
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    with Mode():
+        linear(x, w)
+    assert torch.nn.functional.linear in seen
+    assert type(linear(x.as_subclass(Sub), w)) is Sub
+    weight = torch.nn.Parameter(w)
+    linear(x, weight).backward(t[:, :48])
+    assert weight.grad is not None and not launched
+    if M < 256:
+        with monkeypatch.context() as m:
+            m.setattr(torch, "is_autocast_enabled", lambda device: True)
+            m.setattr(torch, "get_autocast_dtype", lambda device: torch.float16)
+            linear(x, w)
+        assert not launched
+    torch.set_default_device("cpu")
+    try:
+        linear(x, w)
+    finally:
+        torch.set_default_device(None)
+    with torch.no_grad():
+        linear(x, weight)
+    assert launched == ["dd_linear" if M <= 64 else "dd_gemm_bf16"] * 2
+
+
 def test_op_counters_are_not_shared(monkeypatch):
     """Calls on two streams, and calls of two graph captures, never get the same counters (calls that
     overlap would race on them); one stream, and one capture on one stream, keeps its own."""
