@@ -12,9 +12,12 @@
 #include <hipblaslt/hipblaslt-ext.hpp>
 #include <hipblaslt/hipblaslt.h>
 
+#include <algorithm>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "api.h"
@@ -23,6 +26,7 @@ namespace dd {
 namespace {
 
 constexpr int MAX_DEV = 16;
+constexpr size_t MAX_SHAPES = 256;   // shapes kept
 constexpr int NCAND = 16;            // heuristic candidates listed for the tuning tool
 
 std::mutex g_mu;
@@ -46,10 +50,17 @@ struct Desc {
 // What a (device, M, N, K, workspace) runs: the descriptors and, per requested solution index,
 // the algorithm resolved for this problem (the requested one when it supports the problem within
 // the workspace, else the heuristic's first candidate).
+//
+// The first product of a row count is a prompt's time to first token, so what it needs is kept small: a
+// solution's algorithm is looked up once per device, the heuristic is asked only where no named solution
+// runs, and a full record loses its least recently used shape, not all. Host time of the first four products
+// (QKV, O, gate/up, down) of an unseen row count, median of 40, us, F.linear / the heuristic asked each time /
+// this: 65 - 255 rows 322 / 378 / 125, 256 - 1,023 367 / 386 / 142, 1,024 - 8,191 385 / 384 / 184; repeated
+// 78 / 68 / 69.
 struct Shape {
+  int dev = 0;
   Desc d;
-  bool have_first = false;
-  hipblasLtMatmulAlgo_t first;
+  unsigned long long used = 0;       // clock of the last use
   std::map<int, hipblasLtMatmulAlgo_t> algo;
 };
 
@@ -91,23 +102,24 @@ int shape_of(int M, int N, int K, size_t ws_bytes, hipblasLtHandle_t* h_out, Sha
     if (s != HIPBLAS_STATUS_SUCCESS) return blas_err(s);
   }
   *h_out = g_handle[dev];
-  static std::map<std::tuple<int, int, int, int, size_t>, Shape*> shapes;
+  // never destroyed: at exit hipBLASLt may be gone before it
+  static auto& shapes = *new std::map<std::tuple<int, int, int, int, size_t>, std::unique_ptr<Shape>>;
+  static unsigned long long clock = 0;
   const auto key = std::make_tuple(dev, M, N, K, ws_bytes);
   auto it = shapes.find(key);
   if (it == shapes.end()) {
-    if (shapes.size() >= 256) {              // bounded: drop them all (rebuilt on demand)
-      for (auto& kv : shapes) delete kv.second;
-      shapes.clear();
-    }
-    Shape* ns = new Shape;
+    if (shapes.size() >= MAX_SHAPES)         // bounded: the least recently used goes
+      shapes.erase(std::min_element(shapes.begin(), shapes.end(), [](const auto& a, const auto& b) {
+        return a.second->used < b.second->used;
+      }));
+    std::unique_ptr<Shape> ns(new Shape);
+    ns->dev = dev;
     const int e = make_desc(ns->d, M, N, K, ws_bytes);
-    if (e) {
-      delete ns;
-      return e;
-    }
-    it = shapes.emplace(key, ns).first;
+    if (e) return e;
+    it = shapes.emplace(key, std::move(ns)).first;
   }
-  *out = it->second;
+  it->second->used = ++clock;
+  *out = it->second.get();
   return 0;
 }
 
@@ -124,37 +136,42 @@ int candidates(hipblasLtHandle_t h, const Desc& d, int max,
   return 0;
 }
 
+// The algorithm of solution index `solution`, if it runs the shape within the workspace; g_mu held.
+bool named(hipblasLtHandle_t h, const Shape& sh, int solution, size_t ws_bytes, hipblasLtMatmulAlgo_t* out) {
+  static std::map<std::pair<int, int>, hipblasLtMatmulAlgo_t> known;   // by device and index
+  const auto key = std::make_pair(sh.dev, solution);
+  auto it = known.find(key);
+  if (it == known.end()) {
+    std::vector<int> idx{solution};
+    std::vector<hipblasLtMatmulHeuristicResult_t> res;
+    if (hipblaslt_ext::getAlgosFromIndex(h, idx, res) != HIPBLAS_STATUS_SUCCESS || res.empty()) return false;
+    if (known.size() >= MAX_SHAPES) known.clear();
+    it = known.emplace(key, res[0].algo).first;
+  }
+  const float alpha = 1.f, beta = 0.f;
+  size_t need = 0;
+  *out = it->second;
+  return hipblaslt_ext::matmulIsAlgoSupported(h, sh.d.op, &alpha, sh.d.a, sh.d.b, &beta, sh.d.c, sh.d.c, *out,
+                                              need) == HIPBLAS_STATUS_SUCCESS &&
+         need <= ws_bytes;
+}
+
 // The algorithm a (shape, solution) pair runs; g_mu held.
 int resolve(hipblasLtHandle_t h, Shape& sh, int solution, size_t ws_bytes,
             const hipblasLtMatmulAlgo_t** out) {
   auto it = sh.algo.find(solution);
-  if (it != sh.algo.end()) {
-    *out = &it->second;
-    return 0;
-  }
-  if (!sh.have_first) {
-    std::vector<hipblasLtMatmulHeuristicResult_t> cand;
-    const int e = candidates(h, sh.d, 1, cand);
-    if (e) return e;
-    sh.first = cand[0].algo;
-    sh.have_first = true;
-  }
-  hipblasLtMatmulAlgo_t pick = sh.first;
-  if (solution >= 0) {
-    std::vector<int> idx{solution};
-    std::vector<hipblasLtMatmulHeuristicResult_t> res;
-    if (hipblaslt_ext::getAlgosFromIndex(h, idx, res) == HIPBLAS_STATUS_SUCCESS && !res.empty()) {
-      const float alpha = 1.f, beta = 0.f;
-      size_t need = 0;
-      hipblasLtMatmulAlgo_t a = res[0].algo;
-      if (hipblaslt_ext::matmulIsAlgoSupported(h, sh.d.op, &alpha, sh.d.a, sh.d.b, &beta, sh.d.c,
-                                               sh.d.c, a, need) == HIPBLAS_STATUS_SUCCESS &&
-          need <= ws_bytes)
-        pick = a;
+  if (it == sh.algo.end()) {
+    hipblasLtMatmulAlgo_t pick;
+    if (solution < 0 || !named(h, sh, solution, ws_bytes, &pick)) {
+      std::vector<hipblasLtMatmulHeuristicResult_t> cand;
+      const int e = candidates(h, sh.d, 1, cand);
+      if (e) return e;
+      pick = cand[0].algo;
     }
+    if (sh.algo.size() >= 64) sh.algo.clear();
+    it = sh.algo.emplace(solution, pick).first;
   }
-  if (sh.algo.size() >= 64) sh.algo.clear();
-  *out = &sh.algo.emplace(solution, pick).first->second;
+  *out = &it->second;
   return 0;
 }
 
@@ -186,17 +203,8 @@ DD_API int dd_gemm_bf16_supported(int M, int N, int K, size_t ws_bytes, int solu
   hipblasLtHandle_t h = nullptr;
   Shape* sh = nullptr;
   if (shape_of(M, N, K, ws_bytes, &h, &sh)) return 0;
-  std::vector<int> idx{solution};
-  std::vector<hipblasLtMatmulHeuristicResult_t> res;
-  if (hipblaslt_ext::getAlgosFromIndex(h, idx, res) != HIPBLAS_STATUS_SUCCESS || res.empty()) return 0;
-  const float alpha = 1.f, beta = 0.f;
-  size_t need = 0;
-  hipblasLtMatmulAlgo_t a = res[0].algo;
-  return hipblaslt_ext::matmulIsAlgoSupported(h, sh->d.op, &alpha, sh->d.a, sh->d.b, &beta, sh->d.c,
-                                              sh->d.c, a, need) == HIPBLAS_STATUS_SUCCESS &&
-                 need <= ws_bytes
-             ? 1
-             : 0;
+  hipblasLtMatmulAlgo_t algo;
+  return named(h, *sh, solution, ws_bytes, &algo) ? 1 : 0;
 }
 
 DD_API int dd_gemm_bf16_solutions(int M, int N, int K, size_t ws_bytes, int* out, int max) {

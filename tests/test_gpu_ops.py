@@ -545,6 +545,22 @@ def test_attn_streams_and_graphs_at_once(cuda):
             assert all(torch.equal(o, alone[i]) for o in out)
 
 
+def test_gemm_record_past_its_bound(cuda):
+    """More shapes than the product's record holds (256), an older one in use all along, with no named
+    solution, the table's, and one that the library does not know: exact products each time, and the same
+    choice after a shape has been dropped and comes again."""
+    hip = _hip(fake_engine(nh=8, nkv=2, hd=128))
+    from dryft_amd.hipops import load_gemm_table
+    sols = (-1, load_gemm_table()[2560, 4096][0][1], 1 << 30)
+    g = torch.Generator().manual_seed(5)
+    x = torch.randint(-1, 2, (400, 64), generator=g).to(BF).cuda()
+    w = torch.randint(-1, 2, (48, 64), generator=g).to(BF).cuda()
+    ref = (x.float() @ w.float().t()).to(BF)                # |sum| <= 64: exact in bf16
+    for M in (*range(65, 345), 66, 200):
+        assert torch.equal(hip._gemm_lib(x[:M], w, sols[M % 3]), ref[:M]), M
+        assert torch.equal(hip._gemm_lib(x[:65], w, sols[M % 3]), ref[:65]), M
+
+
 # ------------------------------------------------------------------------ argmax
 def test_argmax_rules_and_pos(cuda):
     from dryft_amd.hipops import HipOps
