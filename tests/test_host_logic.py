@@ -88,6 +88,27 @@ def test_qkv_head_grouped_order(nh, nkv):
     assert torch.equal(FusedStep.qkv_natural(grouped, nh, nkv).view(-1), torch.arange(n))
 
 
+def test_gemm_table_is_nowhere_much_slower_than_the_heuristic():
+    """By its own timings the committed table's entries are at most 5% (and a timing's last digit) slower
+    than the heuristic's first candidate, at three row counts of each entry's range and at the row counts
+    between grid points that it records; the lookup takes the entry of the range."""
+    import json
+    from dryft_amd import hipops
+    with open(hipops.GEMM_TABLE) as f:
+        doc = json.load(f)
+    table = hipops.load_gemm_table()
+    for c in doc["check"].values():
+        assert c["table_ms"] <= 1.06 * c["heuristic_first_ms"], c
+    for key, rows in doc["shapes"].items():
+        n, k = (int(v) for v in key.split("x"))
+        assert [m for m, _ in rows] == doc["grid"]
+        for (m, sol), prev in zip(rows, [16] + doc["grid"]):
+            t = doc["timing_ms"][key][str(m)]
+            assert all(a <= 1.05 * b + 2e-4 for a, b in zip(t["table"], t["heuristic_first"])), (key, m, t)
+            assert {hipops.gemm_solution(table, n, k, v) for v in (prev + 1, m)} == {sol}
+        assert hipops.gemm_solution(table, n, k, 10 ** 6) == rows[-1][1]
+
+
 class FakeLib:
     """The library's side of HipOps on the CPU: sizes and choices as the library gives them, and the names
     of the kernels that would have been launched."""
