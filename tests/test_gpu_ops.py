@@ -167,14 +167,18 @@ def weights():
     return {k: (torch.randn(n, kk, generator=g) * 0.02).to(BF) for k, (n, kk) in SHAPES.items()}
 
 
+# The real widths run the streaming kernels (linear.hip); with 8 columns less K is no multiple of 64, which is
+# the GEMV's (gemv.hip).
+@pytest.mark.parametrize("cut", [0, 8])
 @pytest.mark.parametrize("name", list(SHAPES))
-def test_gemv_real_shapes(small, weights, name):
+def test_linear_real_shapes(small, weights, name, cut):
     tor, hip, _ = small
-    w = weights[name]
+    w = weights[name][:, :weights[name].shape[1] - cut].contiguous()
     wg = w.cuda()
     g = torch.Generator().manual_seed(2)
     for M in (1, 4, 8, 16):
         x = torch.randn(M, w.shape[1], generator=g).to(BF)
+        assert hip._linear_ok(x.cuda(), wg) == (cut == 0) and hip._gemv_ok(x.cuda(), wg)
         got = hip.linear(x.cuda(), wg)
         close(got, tor.linear(x, w))
         # fp64 bound: |err| <= bf16 half-ulp of the output + fp32 accumulation error (a few
@@ -188,42 +192,64 @@ def test_gemv_real_shapes(small, weights, name):
 @pytest.mark.parametrize("M,N", [(1, 65576), (8, 65576), (13, 65576), (16, 65576), (16, 40008)])
 def test_gemv_multi_tile_exact(small, M, N):
     """N = 65,576 (4,099 tiles of 16 rows, not a multiple of 64 rows) at M >= 8 takes the
-    unsplit kernel with four W tiles per workgroup (M = 1: one tile); N = 40,008 (2,501 tiles)
-    takes it with two. Integer x and W in [-3, 3] and K = 512 keep every fp32 partial sum exact
-    in any order, so the one rounding is the bf16 store: the fp64 product rounded to bf16 is the
-    exact answer, bit for bit."""
+    unsplit GEMV with four W tiles per workgroup (M = 1: one tile); N = 40,008 (2,501 tiles)
+    takes it with two. Integer x and W in [-3, 3] and K = 520 (no multiple of 64: not the streaming
+    kernel's) keep every fp32 partial sum exact in any order, so the one rounding is the bf16 store:
+    the fp64 product rounded to bf16 is the exact answer, bit for bit."""
     _, hip, _ = small
-    K = 512
+    K = 520
     g = torch.Generator().manual_seed(40 + M)
     x = torch.randint(-3, 4, (M, K), generator=g).to(BF)
     w = torch.randint(-3, 4, (N, K), generator=g).to(BF)
+    assert not hip._linear_ok(x.cuda(), w.cuda())
     got = hip.linear(x.cuda(), w.cuda()).cpu()
     exp = (x.double() @ w.double().T).to(BF)
     assert torch.equal(got, exp)
 
 
-def test_gate_up_silu_real(small, weights):
+@pytest.mark.parametrize("cut", [0, 8])
+def test_gate_up_silu_real(small, weights, cut):
     tor, hip, _ = small
-    w = weights["gate_up"]
+    w = weights["gate_up"][:, :2560 - cut].contiguous()
     g = torch.Generator().manual_seed(3)
     for M in (1, 16):
-        x = torch.randn(M, 2560, generator=g).to(BF)
+        x = torch.randn(M, 2560 - cut, generator=g).to(BF)
+        assert hip._linear_ok(x.cuda(), w.cuda()) == (cut == 0)
         close(hip.gate_up_silu(x.cuda(), w.cuda()), tor.gate_up_silu(x, w))
 
 
+@pytest.mark.parametrize("cut", [0, 8])
 @pytest.mark.parametrize("name", ["o", "down"])
-def test_linear_add_norm_real(small, weights, name):
+def test_linear_add_norm_real(small, weights, name, cut):
     tor, hip, _ = small
-    w = weights[name]
+    w = weights[name][:, :weights[name].shape[1] - cut].contiguous()
     g = torch.Generator().manual_seed(4)
     lnw = (1 + 0.02 * torch.randn(2560, generator=g)).to(BF)
     for M in (1, 16):
         x = torch.randn(M, w.shape[1], generator=g).to(BF)
         h = torch.randn(M, 2560, generator=g).to(BF)
+        assert hip._linear_ok(x.cuda(), w.cuda()) == (cut == 0)
         hn, y = hip.linear_add_norm(x.cuda(), w.cuda(), h.cuda(), lnw.cuda())
         rh, ry = tor.linear_add_norm(x, w, h, lnw)
         close(hn, rh)
         close(y, ry)
+
+
+# the GEMV family (K % 64 != 0) at one tile and a ragged last one, splits of K, and 1 to 16 rows
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("N,K", [(8, 72), (72, 200), (1000, 1032), (2560, 2568)])
+def test_gemv_family_exact(small, M, N, K):
+    """x and W of -1, 0, 1: whole-number sums below 256, exact in fp32 in any order and in bf16, through
+    the plain product, SiLU * up and the residual add + norm."""
+    hip = small[1]
+    g = torch.Generator().manual_seed(M * 7 + N)
+    x = torch.randint(-1, 2, (M, K), generator=g).to(BF)
+    w = torch.randint(-1, 2, (N, K), generator=g).to(BF)
+    ref = x.float() @ w.float().t()
+    assert ref.abs().max() < 256
+    assert hip._gemv_ok(x.cuda(), w.cuda()) and not hip._linear_ok(x.cuda(), w.cuda())
+    assert torch.equal(hip.linear(x.cuda(), w.cuda()).float().cpu(), ref)
+    _epilogues_exact(hip, x, w, ref, g)
 
 
 @pytest.mark.parametrize("M", [17, 64, 65, 300])
@@ -256,10 +282,32 @@ def test_linear_keeps_what_only_f_linear_takes(small, M):
         assert a.data_ptr() != b.data_ptr()
 
 
-# rows at the edges of the 16-row tiles; N and K at a ragged last tile, tiles of 1 / 2 / 4 / 5 / 8 weight
-# tiles, K split over workgroups (few outputs, many rows) and every stage width
+def _epilogues_exact(hip, x, w, ref, g):
+    """SiLU * up and the residual add + norm of a product whose values `ref` are whole numbers below 256."""
+    M, N = ref.shape
+    if N % 2 == 0:
+        gu, up = ref.chunk(2, -1)
+        want = (torch.nn.functional.silu(gu).to(BF).float() * up).to(BF).float()
+        got = hip.gate_up_silu(x.cuda(), w.cuda()).cpu().float()
+        # silu to one bf16 ulp (another expf): 2^-7 at most; one more from the rounding of the product
+        assert ((got - want).abs() <= 2 ** -6 * want.abs() + 1e-30).all()
+    if N <= 4096:
+        h = torch.randint(-64, 65, (M, N), generator=g).to(BF)
+        lnw = torch.ones(N, dtype=BF)
+        hn, y = hip.linear_add_norm(x.cuda(), w.cuda(), h.cuda(), lnw.cuda())
+        want = (h.float() + ref).to(BF).float()
+        assert torch.equal(hn.float().cpu(), want)
+        norm = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + hip.e.eps)
+        # one rounding of the fp32 norm to bf16 (half an ulp: 2^-9), doubled for its own fp32 sum
+        assert ((y.float().cpu() - norm).abs() <= 2 ** -8 * norm.abs() + 1e-30).all()
+
+
+# rows at the edges of the 16-row tiles; N and K at a ragged last tile, K split over workgroups (few outputs,
+# many rows), every stage width, and on 256 CUs (plain, SiLU) tiles of 1 (72 .. 2560), 2 (6144), 4 (12008), 5
+# (20002, 40000) and 8 weight tiles (65576; SiLU 24578)
 @pytest.mark.parametrize("M", [1, 16, 17, 48, 64])
-@pytest.mark.parametrize("N,K", [(72, 256), (1000, 192), (2560, 1024), (6144, 128), (20002, 64), (40000, 128)])
+@pytest.mark.parametrize("N,K", [(72, 256), (1000, 192), (2560, 1024), (6144, 128), (12008, 64), (20002, 64), (24578, 64),
+                                 (40000, 128), (65576, 64)])
 def test_streamed_linear_exact(small, M, N, K):
     """x and W of -1, 0, 1: every product sum is a whole number of at most K <= 1024 with |sum| < 256
     (a random walk), exact in fp32 in any order and in bf16."""
@@ -271,45 +319,21 @@ def test_streamed_linear_exact(small, M, N, K):
     assert ref.abs().max() < 256
     assert hip._linear_ok(x.cuda(), w.cuda())
     assert torch.equal(hip.linear(x.cuda(), w.cuda()).float().cpu(), ref)
-    if N % 2 == 0:
-        gu, up = ref.chunk(2, -1)
-        want = (torch.nn.functional.silu(gu).to(torch.bfloat16).float() * up).to(torch.bfloat16)
-        got = hip.gate_up_silu(x.cuda(), w.cuda()).cpu().float()
-        # silu to one bf16 ulp (another expf): 2^-7 at most; one more from the rounding of the product
-        assert ((got - want.float()).abs() <= 2 ** -6 * want.float().abs() + 1e-30).all()
-    if N <= 4096:
-        h = torch.randint(-64, 65, (M, N), generator=g).to(torch.bfloat16)
-        lnw = torch.ones(N, dtype=torch.bfloat16)
-        hn, y = hip.linear_add_norm(x.cuda(), w.cuda(), h.cuda(), lnw.cuda())
-        want = (h.float() + ref).to(torch.bfloat16).float()
-        assert torch.equal(hn.float().cpu(), want)
-        norm = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + hip.e.eps)
-        assert ((y.float().cpu() - norm).abs() <= 2 ** -8 * norm.abs() + 1e-30).all()
+    _epilogues_exact(hip, x, w, ref, g)
 
 
-# above 64 rows: the edges of the 32-row steps and of the ranges of SiLU (96) and the sums (128), a ragged last tile
+# above 64 rows: the edges of the 32-row steps and of the ranges of SiLU (96) and the sums (128), a ragged last
+# tile, SiLU with 8 weight tiles (24578)
 @pytest.mark.parametrize("M", [65, 80, 96, 97, 128, 129])
-@pytest.mark.parametrize("N,K", [(72, 256), (1000, 192), (2560, 1024), (20002, 64), (40000, 128)])
+@pytest.mark.parametrize("N,K", [(72, 256), (1000, 192), (2560, 1024), (20002, 64), (24578, 64), (40000, 128)])
 def test_streamed_epilogues_exact(small, M, N, K):
     """The products of test_streamed_linear_exact (whole numbers below 256) through the epilogues."""
-    hip = small[1]
     g = torch.Generator().manual_seed(M * 7 + N)
     x = torch.randint(-1, 2, (M, K), generator=g).to(BF)
     w = torch.randint(-1, 2, (N, K), generator=g).to(BF)
     ref = x.float() @ w.float().t()
     assert ref.abs().max() < 256
-    gu, up = ref.chunk(2, -1)
-    want = (torch.nn.functional.silu(gu).to(BF).float() * up).to(BF).float()
-    got = hip.gate_up_silu(x.cuda(), w.cuda()).cpu().float()
-    assert ((got - want).abs() <= 2 ** -6 * want.abs() + 1e-30).all()     # two bf16 roundings, as above
-    if N <= 4096:
-        h = torch.randint(-64, 65, (M, N), generator=g).to(BF)
-        lnw = torch.ones(N, dtype=BF)
-        hn, y = hip.linear_add_norm(x.cuda(), w.cuda(), h.cuda(), lnw.cuda())
-        want = (h.float() + ref).to(BF).float()
-        assert torch.equal(hn.float().cpu(), want)
-        norm = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + hip.e.eps)
-        assert ((y.float().cpu() - norm).abs() <= 2 ** -8 * norm.abs() + 1e-30).all()
+    _epilogues_exact(small[1], x, w, ref, g)
 
 
 def test_linear_dtype_and_layout_fallback(small):

@@ -170,7 +170,7 @@ def test_attn_prefill_packed(cuda, lens, NH, NKV, cap):
     print(f"lens={lens} G={NH // NKV}: max|out - fp64| {d:.3g}")
 
 
-def test_attn_prefill_dma_equals_register_staging(cuda):
+def test_attn_prefill_capacity_changes_no_bit(cuda):
     """The cache's capacity (here a multiple of the key block and not) does not change a bit: the same
     prompts in a cache of 256 and of 264 slots give identical results (and the fp64 bound holds)."""
     lens, NH, NKV = (1, 31, 32, 33, 200, 256), 32, 8
@@ -186,15 +186,49 @@ def test_attn_prefill_dma_equals_register_staging(cuda):
     vc2 = torch.cat([vc, torch.randn(B, NKV, 8, HD, generator=g).to(BF)], dim=2)
     ss = torch.tensor(starts, dtype=torch.int32).cuda()
     qg = q.cuda()
-    dma = hip.attn_prefill_packed(qg, kc.cuda(), vc.cuda(), ss, B, T)
-    reg = hip.attn_prefill_packed(qg, kc2.cuda(), vc2.cuda(), ss, B, T)
-    assert torch.equal(dma, reg)
+    out = hip.attn_prefill_packed(qg, kc.cuda(), vc.cuda(), ss, B, T)
+    assert torch.equal(out, hip.attn_prefill_packed(qg, kc2.cuda(), vc2.cuda(), ss, B, T))
     ref = _attn_ref_fp64(q, kc, vc, lens, starts, NH, NKV)
-    assert (dma.double().cpu() - ref).abs().max().item() < 0.02
+    assert (out.double().cpu() - ref).abs().max().item() < 0.02
     last = torch.tensor(starts[1:]) - 1
     for k, v in ((kc, vc), (kc2, vc2)):
         ol = hip.attn_prefill_packed(qg[last].contiguous(), k.cuda(), v.cuda(), ss, B, T, last_only=True)
-        assert torch.equal(ol, dma[last.cuda()])
+        assert torch.equal(ol, out[last.cuda()])
+
+
+# G = 4 and a mean of 4,096 tokens or more: the 8-wave kernel. Lengths at the edges of its 64-token tiles and
+# 64-key blocks, a mean of exactly 4,096, a short prompt beside a long one
+@pytest.mark.parametrize("lens,NH", [((4096,), 4), ((4097,), 8), ((4159, 4161), 4), ((8160, 32), 4), ((8150, 63), 8)])
+def test_attn_prefill_long_prompts(cuda, lens, NH):
+    """Sampled rows of every prompt within 0.02 of the float64 loop, and all of them the bits of the 4-wave
+    kernel, which takes the same prompts when many short ones lower the batch's mean length."""
+    NKV, B, cap = NH // 4, len(lens), max(lens) + 5
+    hip = _hip(fake_engine(nh=NH, nkv=NKV, hd=HD))
+    starts = _starts(lens)
+    T = starts[-1]
+    assert T // B >= 4096
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(T, NH, HD, generator=g).to(BF)
+    kc = torch.randn(B, NKV, cap, HD, generator=g).to(BF)       # noise past each prompt's length
+    vc = torch.randn(B, NKV, cap, HD, generator=g).to(BF)
+    qg, kg, vg = q.cuda(), kc.cuda(), vc.cuda()
+    out = hip.attn_prefill_packed(qg, kg, vg, torch.tensor(starts, dtype=torch.int32).cuda(), B, T)
+    assert torch.equal(out, hip.attn_prefill_packed(qg, kg, vg, torch.tensor(starts, dtype=torch.int32).cuda(), B, T))
+    for b, n in enumerate(lens):
+        rows = torch.tensor(sorted({p for e in (0, 31, 32, 63, 64, n // 2, n - 1) for p in (e, e + 1)
+                                    if p < n} | set(range(0, n, 257))))
+        for h in range(NH):
+            s = q[starts[b] + rows, h].double() @ kc[b, h // 4, :n].double().T * HD ** -0.5
+            s = s.masked_fill(torch.arange(n)[None] > rows[:, None], float("-inf"))
+            ref = torch.softmax(s, -1) @ vc[b, h // 4, :n].double()
+            d = (out.view(T, NH, HD)[starts[b] + rows.cuda(), h].double().cpu() - ref).abs().max().item()
+            assert d < 0.02, (b, h, d)
+    more = 3 * B                                                # prompts of one token
+    small = [torch.cat([t, torch.zeros(more, NKV, cap, HD, dtype=BF, device="cuda")]) for t in (kg, vg)]
+    ss = torch.tensor(starts + [T + i + 1 for i in range(more)], dtype=torch.int32).cuda()
+    assert (T + more) // (B + more) < 4096
+    packed = hip.attn_prefill_packed(torch.cat([qg, qg[:more]]), *small, ss, B + more, T + more)
+    assert torch.equal(packed[:T], out)
 
 
 @pytest.mark.parametrize("lens,NH", [((130, 65, 200), 32), ((4165,), 4)])
