@@ -307,13 +307,13 @@ def _time(torch, fn, reps):
     return e0.elapsed_time(e1) / reps * 1e-3
 
 
-def micro_gemv(torch, eng):
-    """the per-op skinny GEMV kernel (dd_gemv, MFMA, in-launch split-K) at the five
-    Qwen3-4B projection shapes and M in {1, 4, 8, 16}; bf16 weights N(0, 0.02), x N(0, 1).
+def micro_linear(torch, eng):
+    """the per-op skinny linear kernel (dd_linear: weights streamed through LDS, MFMA) at
+    the five Qwen3-4B projection shapes and M in {1, 4, 8, 16}; bf16 weights N(0, 0.02), x N(0, 1).
     Bytes per launch = N K 2 + M K 2 + M N 2. `us` / `GBps`: the op as generation runs it, inside
     a captured hipGraph (10 calls per graph, replayed; GPU time per call). `us_eager`: the same
-    op called from Python, which the host's per-call work (two tensor allocations, the ctypes
-    call) bounds at ~12 us whatever the shape."""
+    op called from Python, which the host's per-call work (a tensor allocation, the ctypes call)
+    bounds at ~8 us whatever the shape."""
     ops = eng.ops.f if hasattr(eng.ops, "f") else eng.ops
     H, I, V = eng.cfg["hidden_size"], eng.cfg["intermediate_size"], eng.cfg["vocab_size"]
     shapes = {"qkv": ((eng.nh + 2 * eng.nkv) * eng.hd, H), "o": (H, eng.nh * eng.hd),
@@ -331,7 +331,7 @@ def micro_gemv(torch, eng):
             side = torch.cuda.Stream()
             side.wait_stream(torch.cuda.current_stream())
             with torch.cuda.stream(side):
-                ops.linear(x, w)                      # workspace and counters outside capture
+                ops.linear(x, w)
             torch.cuda.current_stream().wait_stream(side)
             gr = torch.cuda.CUDAGraph()
             with torch.cuda.graph(gr):
@@ -613,11 +613,11 @@ def main():
                                                 "one-launch step launched alone)")
         except (OSError, ValueError, KeyError):
             extra["configs1"] = None
-        extra["configs1_per_op_gemv"] = dict(micro_gemv(torch, eng),
-                                             path="dd_gemv, the per-op fallback for B > 16 and "
-                                                  "geometries the one-launch step does not take")
-        print(f"[bench] configs[1] per-op dd_gemv {extra['configs1_per_op_gemv']}", file=sys.stderr,
-              flush=True)
+        extra["configs1_per_op_linear"] = dict(micro_linear(torch, eng),
+                                               path="dd_linear, the per-op path for B > 16 and "
+                                                    "geometries the one-launch step does not take")
+        print(f"[bench] configs[1] per-op dd_linear {extra['configs1_per_op_linear']}",
+              file=sys.stderr, flush=True)
 
     roof = step_roofline(ms, bytes_step, B)
     print(f"[bench] roofline {roof}", file=sys.stderr, flush=True)

@@ -37,8 +37,9 @@
 //   O + norm     18.8 / 16.5   19.1 / 16.9   19.6 / 18.5   19.1 / 18.9   19.5 / 19.5   18.0 / 20.9
 //   down + norm  31.0 / 26.2   32.1 / 27.5   34.4 / 26.9   35.6 / 28.3   36.0 / 28.7   32.6 / 31.4
 // so the sums are taken up to 128 rows and SiLU up to 96 (from 129 to 160 rows it is 2 - 7% ahead again,
-// hipBLASLt's time being a staircase of its tile heights: not worth a second range). A different first stage for each workgroup, so that they do not
-// read the same lines of x at once, gained nothing up to 64 rows and cost 0.5 us in O and down above.
+// hipBLASLt's time being a staircase of its tile heights: not worth a second range). A different first
+// stage for each workgroup, so that they do not read the same lines of x at once, gained nothing up to 64
+// rows and cost 0.5 us in O and down above.
 //
 // MFMA 16x16x32: A = 16 weight rows, B = 16 activation rows (x^T), both read from LDS. The 8 waves
 // split a stage into (k-steps of 32) x (weight tiles), and every wave multiplies its weight fragments
@@ -139,8 +140,8 @@ __global__ void __launch_bounds__(THREADS, 1) linear_kernel(const Args a) {
       (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
 
   // ---- DMA side: instruction i of a stage (wave i % 8) fills LDS rows i RPI .. of W, then of x ----
-  // Rows past M, and weight rows past the tile's last, lie outside the buffers' ranges: the hardware
-  // drops those lanes' reads, and the outputs of such rows are not stored. So every wave issues the
+  // Rows past M, and weight rows past the tile's last, lie outside the buffers' ranges: those lanes
+  // fetch nothing and land zeros, and the outputs of such rows are not stored. So every wave issues the
   // same number of loads in every stage, which is what the waits count.
   const rsrc_t xr = make_rsrc(a.x, (unsigned)a.M * a.K * 2);
   const int ni = (Z::NI - wave + 7) / 8;                               // this wave's instructions
@@ -325,7 +326,8 @@ bool plan_for(int mode, int M, int N, int K, Plan& p) {
   }
   const int parts = (nv + 8 * per16 - 1) / (8 * per16);
   p.nv = nv = (nv + parts - 1) / parts;
-  // weight tiles a stage: the narrow stages are deeper, so that they hold as many bytes
+  // weight tiles a stage: the narrow stages are deeper, so that they hold as many bytes. (The sums reach 5
+  // and 8 only with fewer CUs than a whole card's 256, as in its compute partitions: N <= 4096.)
   const int tiles16 = (nv + per16 - 1) / per16;
   p.nt = tiles16 == 1 && p.bmt <= 2 && K % 256 == 0 ? 1
        : tiles16 <= 2 && K % 128 == 0               ? 2

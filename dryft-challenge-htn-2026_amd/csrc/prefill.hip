@@ -370,10 +370,12 @@ flash_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kc, co
 // A query's bits do not depend on the tile or the number of waves.
 //
 // Graph-timed on MI355X, us, with 16 queries per wave and 32-key blocks (the kernel that this one
-// replaced) / 4 waves / 8 waves: 131 tokens 8.2 / 9.3 / 12.2, 512 17.0 / 16.7 / 21.9, 1,000 33.4 / 27.7 /
-// 32.6, 2,048 91.6 / 57.6 / 63.5, 16 prompts of 64 - 2,048 346 / 292 / 302, 4,096 - / 174 / 157, 8,192 770 /
-// 549 / 525 (1.05 PFLOP/s of causal attention; MFMA 52% busy at the 1.9 GHz that the card holds): 8
-// waves from 4,096 tokens per prompt on.
+// replaced) / this one, in turn on one card: 131 tokens 7.2 / 7.9, 512 16.1 / 15.8, 1,000 32.4 / 26.2, 2,048
+// 88 / 55, 16 prompts of 64 - 2,048 459 / 358, 4,096 239 / 146, 8,192 806 / 529 (1.04 PFLOP/s of causal
+// attention, MFMA 53% and VALU 57% busy). The shortest prompts lose: three 64-key blocks one after the
+// other on 40 workgroups, where 72 had five of 32 keys. 4 waves / 8 waves (another card): 512 16.7 / 21.9,
+// 1,000 27.7 / 32.6, 2,048 57.6 / 63.5, 16 prompts 292 / 302, 4,096 174 / 157, 8,192 549 / 525: 8 waves
+// from 4,096 tokens per prompt on.
 //
 // 32x32x16 layouts: S^T lane l holds query l % 32, keys 8 (i / 4) + 4 (l / 32) + i % 4 of 32; those are
 // the keys its P values keep in the P.V contraction, so P never leaves the lane and the V^T operand

@@ -1934,8 +1934,9 @@ __device__ __forceinline__ void attention_phase(const Args& a, Shared& sh, int l
     }
   };
   auto load_v = [&](size_t kvbase, int key0) {
-    // V streams past the caches (whole 1 KB per load: 416.0 -> 411.0 us for a four-layer step at B = 16 and a mean
-    // context of 1,500, one sequence unchanged); K, read 64 bytes of a line at a time, does not (one sequence 335.7 -> 337.7).
+    // V streams past the caches (whole 1 KB per load: a four-layer step at B = 16 and a mean context of 1,500
+    // 416.3 -> 410.6 us on one card, 418.0 -> 416.1 on another, one sequence unchanged); K, read 64 bytes of a
+    // line at a time, does not (one sequence 335.7 -> 337.7).
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
       const int cc = it * 64 + lane;

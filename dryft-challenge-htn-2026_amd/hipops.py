@@ -2,17 +2,20 @@
 
 Drop-in for the reference's ``TritonOps`` (engine/fused.py:880-1059): same constructor
 ``HipOps(e, use_gemv=True)``, same methods, same argument meaning, same output layouts, and the
-same fallback contract for inputs the kernels do not take (``F.linear`` for non-bf16,
-non-contiguous or M > BM_MAX inputs, i.e. the prefill's GEMMs run on hipBLASLt; torch for
-non-bf16 prefill). The prefill branch of ``qkv_post`` and ``attn_prefill`` run the HIP prefill
+same fallback contract for inputs the kernels do not take. Products run on the weight-streaming
+kernels up to LIN_MAX rows (LIN_SILU_MAX and LIN_NORM_MAX with an epilogue), on the GEMVs up to
+BM_MAX where K is no multiple of 64, and above those rows on hipBLASLt with the table's solution;
+``F.linear`` keeps non-bf16, non-contiguous and unaligned operands, shapes that do not fit (it
+raises), and above BM_MAX rows what more than the caller takes part in (``_plain``); torch keeps the
+non-bf16 prefill. The prefill branch of ``qkv_post`` and ``attn_prefill`` run the HIP prefill
 kernels; ``qkv_post_packed`` / ``attn_prefill_packed`` take a packed ragged batch (prompt b =
 packed tokens ``seq_start[b] .. seq_start[b+1]-1``) so prompts of different lengths prefill in
 one pass. ``e`` carries ``dev, eps, nh, nkv, hd, cos, sin`` like the reference's engine
 (test_fused.py:20-22).
 
 Every decode-step method calls the C ABI on torch's current stream; outputs and workspaces are
-allocated with ``torch.empty`` (so they come from the graph pool under capture). A nonzero
-status raises ``RuntimeError``.
+allocated with ``torch.empty`` (so they come from the graph pool under capture); arrival counters
+and hipBLASLt workspaces are kept per stream and per graph. A nonzero status raises ``RuntimeError``.
 """
 import bisect
 import ctypes

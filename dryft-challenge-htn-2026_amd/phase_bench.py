@@ -12,7 +12,7 @@ duration of its launches minus the embedding phase's (a gather of M rows: the la
 set-up and exit). Bytes per phase follow configs[1]: N K 2 (weights) + M K 2 (activation) +
 M N 2 (output).
 
-Per-op kernels (``--per-op``): dd_gemv at the five projection shapes and M in 1, 4, 8, 16, then
+Per-op kernels (``--per-op``): dd_linear at the five projection shapes and M in 1, 4, 8, 16, then
 dd_attn_decode at configs[2] (B = 16, ragged contexts U[512, 8192], cap 8192), a few launches
 each, and three 1 GiB streaming reads (the byte counters' calibration), for
 ``rocprofv3 --kernel-trace --stats`` and ``--pmc`` runs.
@@ -105,7 +105,7 @@ def parse_trace(trace_csv, plan, shapes):
 
 
 def per_op(torch, eng, reps=10):
-    """dd_gemv at the configs[1] shapes and dd_attn_decode at configs[2], `reps` launches each
+    """dd_linear at the configs[1] shapes and dd_attn_decode at configs[2], `reps` launches each
     (for the profiler); returns {kernel: us per launch} from HIP events."""
     from dryft_amd._lib import check
     ops = eng.ops.f if hasattr(eng.ops, "f") else eng.ops
@@ -122,7 +122,7 @@ def per_op(torch, eng, reps=10):
                 ops.linear(x, w)
             e1.record()
             e1.synchronize()
-            res[f"dd_gemv {name} M{M}"] = round(e0.elapsed_time(e1) * 1e3 / reps, 2)
+            res[f"dd_linear {name} M{M}"] = round(e0.elapsed_time(e1) * 1e3 / reps, 2)
         del w
     # B = 16, ragged contexts U[512, 8192], cap 8192, 32 q / 8 kv heads
     B, NH, NKV, HD, cap = 16, eng.nh, eng.nkv, eng.hd, 8192
@@ -155,22 +155,22 @@ def per_op(torch, eng, reps=10):
 def parse_per_op(trace_dir, pmc_dirs, shapes, reps=10):
     """Per-kernel figures of a ``--per-op`` run from its rocprofv3 outputs: the kernel trace
     (dispatch durations) and --pmc passes (FETCH_SIZE, WRITE_SIZE in KiB; SQ_VALU_MFMA_BUSY_CYCLES,
-    GRBM_GUI_ACTIVE). Dispatches are matched to the run's launch order (per dd_gemv shape and M:
+    GRBM_GUI_ACTIVE). Dispatches are matched to the run's launch order (per dd_linear shape and M:
     one warm-up and `reps` timed launches; then dd_attn_decode likewise; then three 1 GiB
-    stream reads, whose FETCH_SIZE calibrates the byte counters). Returns rows of
-    {kernel, us, algo_GBps, hbm_GBps, hbm_over_algo, mfma_util}."""
+    stream reads, whose FETCH_SIZE calibrates the byte counters); raises when a kernel has not as many
+    as the run makes. Returns rows of {kernel, us, algo_GBps, hbm_GBps, hbm_over_algo, mfma_util}."""
     import csv
     import glob
 
-    def dispatches(path, name_filter, counter=None):
-        names = (name_filter,) if isinstance(name_filter, str) else name_filter
+    def dispatches(path, name, counter=None, want=None):
         out = []
         with open(path) as f:
             for r in csv.DictReader(f):
-                if (any(n in r["Kernel_Name"] for n in names)
-                        and (counter is None or r["Counter_Name"] == counter)):
+                if name in r["Kernel_Name"] and (counter is None or r["Counter_Name"] == counter):
                     v = float(r["Counter_Value"]) if counter else (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
                     out.append((int(r.get("Dispatch_Id") or r.get("Correlation_Id") or 0), v))
+        if want is not None and len(out) != want:
+            raise SystemExit(f"{path}: {len(out)} dispatches of {name}, a --per-op run makes {want}")
         out.sort()
         return [v for _, v in out]
 
@@ -182,27 +182,24 @@ def parse_per_op(trace_dir, pmc_dirs, shapes, reps=10):
             names = {r["Counter_Name"] for r in csv.DictReader(fh)}
         for c in names:
             pmc[c] = f
-    cal = dispatches(pmc["FETCH_SIZE"], "stream_read_kernel", "FETCH_SIZE")
+    cal = dispatches(pmc["FETCH_SIZE"], "stream_read_kernel", "FETCH_SIZE", 3)
     scale = (1 << 30) / 1024 / (sum(cal) / len(cal))         # true KiB / counted KiB
     rows = []
-    # dd_gemv launches gemv_kernel, or gemv_multi_kernel (several W tiles per workgroup) for
-    # unsplit shapes at M >= 8
-    kinds = [(("gemv_kernel", "gemv_multi_kernel"), [(n, m) for n in shapes for m in (1, 4, 8, 16)]),
-             ("attn_decode_kernel", [("configs[2]", 16)])]
+    kinds = [("linear_kernel", [(n, m) for n in shapes for m in (1, 4, 8, 16)]),
+             ("attn_stream_kernel", [("configs[2]", 16)])]
     for kern, cases in kinds:
-        us = dispatches(trace, kern)
-        fetch = dispatches(pmc["FETCH_SIZE"], kern, "FETCH_SIZE")
-        write = dispatches(pmc["WRITE_SIZE"], kern, "WRITE_SIZE")
-        busy = dispatches(pmc["SQ_VALU_MFMA_BUSY_CYCLES"], kern, "SQ_VALU_MFMA_BUSY_CYCLES")
-        gui = dispatches(pmc["GRBM_GUI_ACTIVE"], kern, "GRBM_GUI_ACTIVE")
+        want = len(cases) * (reps + 1)
+        us = dispatches(trace, kern, None, want)
+        fetch, write, busy, gui = (dispatches(pmc[c], kern, c, want) for c in (
+            "FETCH_SIZE", "WRITE_SIZE", "SQ_VALU_MFMA_BUSY_CYCLES", "GRBM_GUI_ACTIVE"))
         for i, (name, M) in enumerate(cases):
             sl = slice(i * (reps + 1) + 1, (i + 1) * (reps + 1))
             mean = lambda v: sum(v[sl]) / len(v[sl])
             t = mean(us)
-            if "gemv_kernel" in kern:
+            if kern == "linear_kernel":
                 N, K = shapes[name]
                 algo = N * K * 2 + M * K * 2 + M * N * 2
-                label = f"dd_gemv {name} {N}x{K} M={M}"
+                label = f"dd_linear {name} {N}x{K} M={M}"
             else:
                 import torch
                 ctx = torch.randint(512, 8193, (16,), generator=torch.Generator().manual_seed(2))

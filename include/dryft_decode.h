@@ -124,7 +124,10 @@ int dd_qkv_post_decode(const void* qkv, const void* qn, const void* kn, const vo
  * q: [B, NKV, W, G, HD] (dd_qkv_post_decode layout); kc/vc: [B, NKV, cap, HD] (zero-initialised);
  * query row (b, s) sees keys 0 .. pos[b*pos_stride] + s. out: [B*W, NH*HD].
  * chunk: keys per split (multiple of 32; <= 0 picks dd_attn_chunk); with dd_attn_chunk's own value
- * and W*G <= 4, B <= 512 the batch is dealt in equal shares instead. ws: dd_attn_ws_bytes bytes;
+ * and W*G <= 4, B <= 512 the batch is dealt in equal shares instead: the partials of any length then
+ * use ws and counters, and a row's last bits depend on the lengths of the other rows too (the same batch
+ * gives the same bits; a chunk other than dd_attn_chunk's keeps them to B, NKV and cap).
+ * ws: dd_attn_ws_bytes bytes;
  * counters: B*NKV ints, zero before the first call (kernels leave them zero).
  * HD must be 128 and W*G <= 32.
  * Replaces TritonOps.attn_decode (fused.py:961-987; kernels fused.py:478-565), reference
