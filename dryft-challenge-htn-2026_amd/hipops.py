@@ -190,9 +190,13 @@ class HipOps:
             kept = self._graph_counters[1]
             c = kept.get(key)
             if c is None or c.numel() < n:
-                fits = n <= COUNTERS and dev == self.err.device
-                c = kept[key] = (self._spare.pop() if fits and self._spare else
-                                 torch.zeros(max(n, COUNTERS), dtype=torch.int32, device=dev))
+                try:
+                    if n > COUNTERS or dev != self.err.device:
+                        raise IndexError
+                    c = self._spare.pop()  # one step: another thread may be capturing too
+                except IndexError:
+                    c = torch.zeros(max(n, COUNTERS), dtype=torch.int32, device=dev)
+                kept[key] = c
             return c
         c = self._counters.get(key)
         if c is None or c.numel() < n:

@@ -191,6 +191,8 @@ def test_products_are_seen_by_what_watches_torch(cpu_ops, monkeypatch, M):
     for mode in ("real", "fake"):
         assert torch.equal(make_fx(lambda a, b: linear(a, b), tracing_mode=mode)(x, w)(t, w), dy)
     assert torch.equal(torch.jit.trace(lambda a: linear(a, w), (x,), check_trace=False)(t), dy)
+    torch._dynamo.reset()
+    assert torch.equal(torch.compile(lambda a, b: linear(a, b), backend="eager", fullgraph=True)(x, w), y)
     with FlopCounterMode(display=False) as flops:
         linear(x, w)
     assert flops.get_total_flops() == 2 * M * 48 * 64
