@@ -180,47 +180,63 @@ int resolve(hipblasLtHandle_t h, Shape& sh, int solution, size_t ws_bytes,
 
 using namespace dd;
 
+// The containers above may run out of memory: nothing throws across the C entries.
+template <class F>
+static int no_throw(int failed, F&& f) {
+  try {
+    return f();
+  } catch (...) {
+    return failed;
+  }
+}
+
 DD_API size_t dd_gemm_ws_bytes(void) { return (size_t)64 << 20; }
 
 DD_API int dd_gemm_bf16(const void* x, const void* w, void* y, int M, int N, int K, void* ws,
                         size_t ws_bytes, int solution, hipStream_t stream) {
   DD_REQUIRE(x && w && y && M >= 1 && N >= 1 && K >= 1);
   DD_REQUIRE(ws_bytes == 0 || ws != nullptr);
-  std::lock_guard<std::mutex> lock(g_mu);
-  hipblasLtHandle_t h = nullptr;
-  Shape* sh = nullptr;
-  int e = shape_of(M, N, K, ws_bytes, &h, &sh);
-  if (e) return e;
-  const hipblasLtMatmulAlgo_t* algo = nullptr;
-  e = resolve(h, *sh, solution, ws_bytes, &algo);
-  if (e) return e;
-  return run(h, sh->d, *algo, x, w, y, ws, ws_bytes, stream);
+  return no_throw((int)hipErrorOutOfMemory, [&]() -> int {
+    std::lock_guard<std::mutex> lock(g_mu);
+    hipblasLtHandle_t h = nullptr;
+    Shape* sh = nullptr;
+    int e = shape_of(M, N, K, ws_bytes, &h, &sh);
+    if (e) return e;
+    const hipblasLtMatmulAlgo_t* algo = nullptr;
+    e = resolve(h, *sh, solution, ws_bytes, &algo);
+    if (e) return e;
+    return run(h, sh->d, *algo, x, w, y, ws, ws_bytes, stream);
+  });
 }
 
 DD_API int dd_gemm_bf16_supported(int M, int N, int K, size_t ws_bytes, int solution) {
   if (!(M >= 1 && N >= 1 && K >= 1 && solution >= 0)) return 0;
-  std::lock_guard<std::mutex> lock(g_mu);
-  hipblasLtHandle_t h = nullptr;
-  Shape* sh = nullptr;
-  if (shape_of(M, N, K, ws_bytes, &h, &sh)) return 0;
-  hipblasLtMatmulAlgo_t algo;
-  return named(h, *sh, solution, ws_bytes, &algo) ? 1 : 0;
+  return no_throw(0, [&]() -> int {
+    std::lock_guard<std::mutex> lock(g_mu);
+    hipblasLtHandle_t h = nullptr;
+    Shape* sh = nullptr;
+    if (shape_of(M, N, K, ws_bytes, &h, &sh)) return 0;
+    hipblasLtMatmulAlgo_t algo;
+    return named(h, *sh, solution, ws_bytes, &algo) ? 1 : 0;
+  });
 }
 
 DD_API int dd_gemm_bf16_solutions(int M, int N, int K, size_t ws_bytes, int* out, int max) {
   if (!(M >= 1 && N >= 1 && K >= 1 && out && max >= 1)) return -1;
-  std::lock_guard<std::mutex> lock(g_mu);
-  hipblasLtHandle_t h = nullptr;
-  Shape* sh = nullptr;
-  int e = shape_of(M, N, K, ws_bytes, &h, &sh);
-  if (e) return -1;
-  std::vector<hipblasLtMatmulHeuristicResult_t> cand;
-  e = candidates(h, sh->d, max < NCAND ? max : NCAND, cand);
-  if (e) return -1;
-  int n = 0;
-  for (auto& c : cand) {
-    if (c.state != HIPBLAS_STATUS_SUCCESS || c.workspaceSize > ws_bytes) continue;
-    out[n++] = hipblaslt_ext::getIndexFromAlgo(c.algo);
-  }
-  return n;
+  return no_throw(-1, [&]() -> int {
+    std::lock_guard<std::mutex> lock(g_mu);
+    hipblasLtHandle_t h = nullptr;
+    Shape* sh = nullptr;
+    int e = shape_of(M, N, K, ws_bytes, &h, &sh);
+    if (e) return -1;
+    std::vector<hipblasLtMatmulHeuristicResult_t> cand;
+    e = candidates(h, sh->d, max < NCAND ? max : NCAND, cand);
+    if (e) return -1;
+    int n = 0;
+    for (auto& c : cand) {
+      if (c.state != HIPBLAS_STATUS_SUCCESS || c.workspaceSize > ws_bytes) continue;
+      out[n++] = hipblaslt_ext::getIndexFromAlgo(c.algo);
+    }
+    return n;
+  });
 }

@@ -33,6 +33,7 @@ def test_validation_rejects_without_launch():
     L = dryft_amd.lib()
     INVALID = 1
     # null pointers
+    assert L.dd_capture_id(None, None) == INVALID
     assert L.dd_gemv(None, None, None, 1, 16, 64, 1, None, None, None) == INVALID
     assert L.dd_rmsnorm(None, None, None, 1, 16, 1e-6, None) == INVALID
     # shape limits checked before any pointer is used (fake, never-dereferenced addresses)
